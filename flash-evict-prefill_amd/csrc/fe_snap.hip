@@ -8,13 +8,24 @@
 //   sum over the W window rows of p                                               (:26-27)
 //
 // The dot products accumulate in FP32 on MFMA and are rounded to the input dtype before
-// the FP32 softmax, as the native-dtype matmul of the reference does. Three kernels:
-//   snap_stats_kernel    per (b, kv head, 32-row tile, key split): partial row max and
-//                        sum of exponentials over the split's keys (lanes hold rows)
-//   snap_combine_kernel  per row: merges the splits into the row max and 1/sum
-//   snap_scores_kernel   per (b, kv head, 64 keys): every window row of the group, p
-//                        summed over rows in-lane (lanes hold keys), / G, one store per key
+// the FP32 softmax, as the native-dtype matmul of the reference does. Two kernels:
+//   snap_stats_kernel    per key block: partial row max and sum of exponentials of every
+//                        window row of the group (lanes hold rows)
+//   snap_scores_kernel   per key block: merges the partials into each row's max and 1/sum,
+//                        then p summed over the rows in-lane (lanes hold keys), / G, one
+//                        store per key
+// Both take the same key blocks in the same order, so the second read of a block's K finds it
+// in the L2 of the XCD that read it first. A window of more than kSnapLdsRows rows per group
+// merges its partials once, in snap_combine_kernel between the two, instead of in every block.
 // No atomics: every score is written once, in a fixed summation order.
+//
+// What bounds it: K is read once from HBM (33.5 MB at N = 32768, 4 KV heads: 7 us) and each
+// logit takes two exponentials (2 x 29 M at 28 heads x 32 rows, 10 us of vector work); launches
+// and the latency of each step make the rest. Layout: a wave keeps the K fragments of its keys in
+// registers and runs over the row tiles, whose Q fragments it reads one tile ahead. (One row tile
+// per wave against a strip of K, 64-thread blocks, read K once per row tile and left a combine
+// kernel of few threads with a serial loop over the strips: 47.6 + 37.2 + 35.0 us at 28/4 heads,
+// N = 32768, D = 128, window 32, against 19.0 + 23.6 us here.)
 #include <math.h>
 #include <string>
 
@@ -24,17 +35,24 @@
 
 namespace fe {
 
+// Waves of a block: KG key groups x (waves / KG) row parts. Above tile dim 128 the K fragments of
+// 64 keys take 128 registers: one wave per SIMD.
+constexpr int snap_waves(int DP) { return DP > 128 ? 4 : 8; }
+constexpr int kSnapChunk = 8;        // row tiles between two merges of the key groups' partials
+constexpr int kSnapLdsRows = 2048;   // rows per group whose statistics a scores block keeps in LDS
+
 struct SnapArgs {
   const u16* q;
   const u16* k;
   float* scores;
-  float2* part;          // [BH][RT][S][32] (max, sum) partials
-  float2* stats;         // [BH][RT][32] (max, 1/sum)
+  float2* part;          // [BH][S][Rp] (max, sum) partials
+  float2* stats;         // [BH][Rp] (max, 1/sum), windows of more than kSnapLdsRows rows
   long long qs[4], ks[4];
   int N, D, G, Hkv, BH;
-  int W, R, RT;          // window rows per head, rows per group (G*W), 32-row tiles
-  int S, tiles_per_split, ntiles;
-  float scale;           // D^-0.5 as float
+  int W, R, RT, Rp;      // window rows per head, rows per group (G*W), 32-row tiles, 32 * RT
+  int S;                 // key blocks per (b, kv head)
+  int KG;                // key groups (of KT 32-key halves) per block
+  float scale_log2;      // D^-0.5 * log2 e
 };
 
 // Row r of a group: head g = r / W of the group, query position N - W + r % W.
@@ -44,165 +62,302 @@ __device__ __forceinline__ void snap_row(const SnapArgs& a, int hkv, int r, int&
   qpos = a.N - a.W + (r - g * a.W);
 }
 
+// The 16 dot products of an accumulator rounded to the input type, in place.
 template <typename E>
-__device__ __forceinline__ float round_logit(float acc) {
-  return E::to_f32((unsigned short)(E::pack2(acc, 0.f) & 0xffffu));
+__device__ __forceinline__ void round_logits(f32x16& x) {
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) {
+    const u32 p = E::pack2(x[i], x[i + 1]);
+    x[i] = E::to_f32((unsigned short)(p & 0xffffu));
+    x[i + 1] = E::to_f32((unsigned short)(p >> 16));
+  }
 }
 
-template <typename E, int DP, int VEC>
-__global__ __launch_bounds__(64) void snap_stats_kernel(const SnapArgs a) {
-  constexpr int NDC = DP / 16;
-  constexpr float NEG_INF = -__builtin_huge_valf();
-  const int lane = threadIdx.x, l32 = lane & 31, hh = lane >> 5;
-  const int s_idx = (int)(blockIdx.x % (unsigned)a.S);
-  const int rest = (int)(blockIdx.x / (unsigned)a.S);
-  const int rt = rest % a.RT, bh = rest / a.RT;
-  const int b = bh / a.Hkv, hkv = bh - b * a.Hkv;
-  const int r = rt * 32 + l32;
-  const bool row_ok = r < a.R;
-  int head = 0, qpos = -1;
-  if (row_ok) snap_row(a, hkv, r, head, qpos);
+// Rows in LDS: DP / 8 16-byte chunks per row, chunk ch of row r at position ch ^ snap_swz(r), so
+// that the 16 lanes of a read phase (one chunk of 16 rows) hit every bank once. Rows come from
+// HBM whole, consecutive lanes on consecutive chunks: read as fragments straight from global
+// memory (32-byte pieces of 32 rows per load, 128 KiB in flight per CU for 32 KiB of L1) they took
+// 41.8 + 34.0 us at 28/4 heads, N = 32768, window 32.
+template <int DP>
+__device__ __forceinline__ int snap_swz(int r) {
+  return DP == 64 ? (r >> 1) & 7 : r & 15;
+}
+template <int DP>
+__device__ __forceinline__ u32x4 snap_frag(const u32x4* rows, int r, int ch) {
+  return rows[r * (DP / 8) + (ch ^ snap_swz<DP>(r))];
+}
 
-  // Q fragments (B operand): query row r, channels 16c + 8h .. +7
-  u32x4 qf[NDC];
-  const u16* qrow = a.q + b * a.qs[0] + head * a.qs[1] + (long long)(row_ok ? qpos : 0) * a.qs[2];
+// The wave's K fragments of keys kb .. kb+31 through its own 32 rows of LDS (zeros past N).
+template <int DP, int VEC>
+__device__ __forceinline__ void snap_load_keys(const SnapArgs& a, const u16* kbase, int kb, u32x4* rows, u32x4 (&f)[DP / 16]) {
+  constexpr int CPR = DP / 8, NL = 32 * CPR / 64;
+  const int lane = threadIdx.x & 63;
+  u32x4 v[NL];
 #pragma unroll
-  for (int c = 0; c < NDC; ++c)
-    qf[c] = row_ok ? load8(qrow, a.qs[3], 16 * c + 8 * hh, a.D, VEC) : (u32x4){0u, 0u, 0u, 0u};
-  const u16* kbase = a.k + b * a.ks[0] + hkv * a.ks[1];
+  for (int j = 0; j < NL; ++j) {
+    const int i = lane + 64 * j, key = kb + i / CPR;
+    const bool ok = key < a.N;
+    v[j] = ok ? load8(kbase + (long long)key * a.ks[2], a.ks[3], 8 * (i % CPR), a.D, VEC) : (u32x4){0u, 0u, 0u, 0u};
+    if (!VEC) __builtin_amdgcn_sched_barrier(0);   // element loads: one chunk's addresses at a time
+  }
+#pragma unroll
+  for (int j = 0; j < NL; ++j) {
+    const int i = lane + 64 * j;
+    rows[(i / CPR) * CPR + ((i % CPR) ^ snap_swz<DP>(i / CPR))] = v[j];
+  }
+  // one wave's LDS operations complete in order: the reads below see the writes above, and the
+  // next call's writes come after these reads
+#pragma unroll
+  for (int c = 0; c < DP / 16; ++c) f[c] = snap_frag<DP>(rows, lane & 31, 2 * c + (lane >> 5));
+}
 
-  float m = NEG_INF, l = 0.f;
-  const int t_lo = s_idx * a.tiles_per_split;
-  const int t_hi = min(a.ntiles, t_lo + a.tiles_per_split);
-  for (int t = t_lo; t < t_hi; ++t) {
-    const int kb = t * 64;
-    f32x16 sacc[2];
+// Row tiles rt0 .. rt0 + kSnapChunk - 1 of the group's query rows into LDS by the whole block
+// (zeros past the last row).
+template <int DP, int VEC, int NT>
+__device__ __forceinline__ void snap_load_rows(const SnapArgs& a, int b, int hkv, int rt0, u32x4* rows) {
+  constexpr int CPR = DP / 8, NL = kSnapChunk * 32 * CPR / NT, U = VEC ? (NL < 8 ? NL : 8) : 1;
+  static_assert(NL % U == 0, "row chunk");
+  for (int j0 = 0; j0 < NL; j0 += U) {
+    if (rt0 * 32 + (NT * j0) / CPR >= a.Rp) break;   // past the last tile
+    u32x4 v[U];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int key = kb + 32 * s + l32;
-      const bool kok = key < a.N;
-      const u16* krow = kbase + (long long)(kok ? key : 0) * a.ks[2];
-      sacc[s] = (f32x16){};
-#pragma unroll
-      for (int c = 0; c < NDC; ++c) {
-        const u32x4 kf = kok ? load8(krow, a.ks[3], 16 * c + 8 * hh, a.D, VEC) : (u32x4){0u, 0u, 0u, 0u};
-        sacc[s] = E::mfma(kf, qf[c], sacc[s]);
-      }
+    for (int u = 0; u < U; ++u) {
+      const int i = (int)threadIdx.x + NT * (j0 + u), r = rt0 * 32 + i / CPR;
+      int head = 0, qpos = 0;
+      if (r < a.R) snap_row(a, hkv, r, head, qpos);
+      v[u] = r < a.R ? load8(a.q + b * a.qs[0] + head * a.qs[1] + (long long)qpos * a.qs[2], a.qs[3], 8 * (i % CPR), a.D, VEC)
+                     : (u32x4){0u, 0u, 0u, 0u};
     }
-    // lanes hold query row r; register i of half s holds key kb + 32s + 8(i/4) + 4h + i%4
-    float x[2][16];
-    float tmax = NEG_INF;
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = kb + 32 * s + 8 * (i >> 2) + 4 * hh + (i & 3);
-        const float v = round_logit<E>(sacc[s][i]) * a.scale;
-        x[s][i] = key <= qpos ? v : NEG_INF;
-        tmax = fmaxf(tmax, x[s][i]);
-      }
-    tmax = half_swap_max(tmax);
-    const float mn = fmaxf(m, tmax);
-    if (mn != NEG_INF) {
-      float sum = 0.f;
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sum += expf(x[s][i] - mn);
-      l = l * expf(m - mn) + half_swap_sum(sum);
-      m = mn;
+    for (int u = 0; u < U; ++u) {
+      const int i = (int)threadIdx.x + NT * (j0 + u);
+      rows[(i / CPR) * CPR + ((i % CPR) ^ snap_swz<DP>(i / CPR))] = v[u];
     }
   }
-  if (hh == 0) a.part[((long long)(bh * a.RT + rt) * a.S + s_idx) * 32 + l32] = make_float2(m, l);
+}
+
+// Position of the group's row r (-1: padding of the last tile).
+__device__ __forceinline__ int snap_qpos(const SnapArgs& a, int r) {
+  return r < a.R ? a.N - a.W + r % a.W : -1;
+}
+
+// exp(scale * x) for x <= 0, a difference of two rounded logits (exact in FP32 unless one is
+// 2^13 times the other): one product by scale * log2 e and v_exp_f32. Against 64 bits the scores
+// are as close as with expf(scale * logit - scale * max): 7.3e-7 to 3.6e-6 relative over ten shapes
+// of 2144 to 54886 keys, the two within 0.5% of each other on each (most of it is logits that FP32
+// sums round the other way).
+__device__ __forceinline__ float snap_exp(const SnapArgs& a, float x) { return fast_exp2(x * a.scale_log2); }
+
+// Merge of two softmax partials (a partial without a visible key: max -inf, sum 0).
+__device__ __forceinline__ void snap_merge(const SnapArgs& a, float& m, float& l, float m2, float l2) {
+  const float mn = fmaxf(m, m2);
+  if (mn != -__builtin_huge_valf()) l = l * snap_exp(a, m - mn) + l2 * snap_exp(a, m2 - mn);
+  m = mn;
+}
+
+template <typename E, int DP, int VEC, int KT>
+__global__ __launch_bounds__(64 * snap_waves(DP)) void snap_stats_kernel(const SnapArgs a) {
+  constexpr int NDC = DP / 16, NW = snap_waves(DP);
+  constexpr float NEG_INF = -__builtin_huge_valf();
+  __shared__ u32x4 rows[kSnapChunk * 32 * (DP / 8)];   // K on the way to registers, then Q
+  __shared__ float2 sm[NW][kSnapChunk * 32];
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wv % a.KG, rp = wv / a.KG, RP = NW / a.KG;
+  const int bh = (int)(blockIdx.x % (unsigned)a.BH), blk = (int)(blockIdx.x / (unsigned)a.BH);
+  const int b = bh / a.Hkv, hkv = bh - b * a.Hkv;
+  const int kb = (blk * a.KG + kg) * 32 * KT;
+  const u16* kbase = a.k + b * a.ks[0] + hkv * a.ks[1];
+
+  u32x4 kf[KT][NDC];                              // K fragments (A operand) of the wave's keys
+#pragma unroll
+  for (int s = 0; s < KT; ++s)
+    snap_load_keys<DP, VEC>(a, kbase, kb + 32 * s, rows + wv * 32 * (DP / 8), kf[s]);
+  __syncthreads();
+  const bool masked = kb + 32 * KT > a.N - a.W;   // some key of the wave is past some row
+  for (int rt0 = 0; rt0 < a.RT; rt0 += kSnapChunk) {
+    snap_load_rows<DP, VEC, 64 * NW>(a, b, hkv, rt0, rows);
+    __syncthreads();
+    for (int rt = rt0 + rp; rt < min(rt0 + kSnapChunk, a.RT); rt += RP) {
+      f32x16 x[KT];
+#pragma unroll
+      for (int c = 0; c < NDC; ++c) {
+        const u32x4 qf = snap_frag<DP>(rows, (rt - rt0) * 32 + l32, 2 * c + hh);
+#pragma unroll
+        for (int s = 0; s < KT; ++s)
+          x[s] = c == 0 ? E::mfma(kf[s][0], qf, (f32x16){}) : E::mfma(kf[s][c], qf, x[s]);
+      }
+      // lanes hold query row rt*32 + l32; register i of half s holds key kb + 32s + 8(i/4) + 4h + i%4
+      float m = NEG_INF, l = 0.f;
+#pragma unroll
+      for (int s = 0; s < KT; ++s) {
+        round_logits<E>(x[s]);
+        if (masked) {
+          const int rel = snap_qpos(a, rt * 32 + l32) - kb - 32 * s - 4 * hh;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) x[s][i] = 8 * (i >> 2) + (i & 3) <= rel ? x[s][i] : NEG_INF;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m = fmaxf(m, x[s][i]);
+      }
+      m = half_swap_max(m);
+      if (m != NEG_INF) {
+#pragma unroll
+        for (int s = 0; s < KT; ++s) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) l += snap_exp(a, x[s][i] - m);
+        }
+      }
+      l = half_swap_sum(l);
+      if (hh == 0) sm[kg][(rt - rt0) * 32 + l32] = make_float2(m, l);
+    }
+    __syncthreads();
+    const int nrows = min(kSnapChunk, a.RT - rt0) * 32;
+    for (int r = tid; r < nrows; r += 64 * NW) {
+      float m = sm[0][r].x, l = sm[0][r].y;
+      for (int g = 1; g < a.KG; ++g) snap_merge(a, m, l, sm[g][r].x, sm[g][r].y);
+      a.part[((long long)bh * a.S + blk) * a.Rp + rt0 * 32 + r] = make_float2(m, l);
+    }
+    __syncthreads();
+  }
+}
+
+// (max, 1/sum) of row r of a group from partials s0, s0 + step, ... of its key blocks; four loads
+// in flight. Every row of the window sees at least key 0.
+__device__ __forceinline__ void snap_merge_parts(const SnapArgs& a, int bh, int r, int s0, int step, float& m, float& l) {
+  const float2* p = a.part + (long long)bh * a.S * a.Rp + r;
+  m = -__builtin_huge_valf();
+  l = 0.f;
+  for (int s = s0; s < a.S; s += 4 * step) {
+    float2 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      v[u] = s + u * step < a.S ? p[(long long)(s + u * step) * a.Rp] : make_float2(-__builtin_huge_valf(), 0.f);
+    float mn = m;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) mn = fmaxf(mn, v[u].x);
+    if (mn != -__builtin_huge_valf()) {
+      l *= snap_exp(a, m - mn);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) l += v[u].y * snap_exp(a, v[u].x - mn);
+    }
+    m = mn;
+  }
 }
 
 __global__ __launch_bounds__(256) void snap_combine_kernel(const SnapArgs a) {
-  const long long row = (long long)blockIdx.x * blockDim.x + threadIdx.x;   // (bh*RT + rt)*32 + i
-  const long long rows = (long long)a.BH * a.RT * 32;
-  if (row >= rows) return;
-  constexpr float NEG_INF = -__builtin_huge_valf();
-  const long long tile = row / 32, i = row - tile * 32;
-  const float2* p = a.part + tile * a.S * 32 + i;
-  float m = NEG_INF;
-  for (int s = 0; s < a.S; ++s) m = fmaxf(m, p[s * 32].x);
-  float l = 0.f;
-  if (m != NEG_INF)
-    for (int s = 0; s < a.S; ++s) {
-      const float2 v = p[s * 32];
-      if (v.x != NEG_INF) l += v.y * expf(v.x - m);
-    }
-  // rows with no visible key (padding rows of the last tile) contribute nothing
-  a.stats[row] = m == NEG_INF ? make_float2(0.f, 0.f) : make_float2(m, 1.f / l);
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long long)a.BH * a.Rp) return;
+  const int bh = (int)(i / a.Rp), r = (int)(i - (long long)bh * a.Rp);
+  float m, l;
+  snap_merge_parts(a, bh, r, 0, 1, m, l);
+  a.stats[i] = make_float2(m, 1.f / l);
 }
 
-template <typename E, int DP, int VEC>
-__global__ __launch_bounds__(64) void snap_scores_kernel(const SnapArgs a) {
-  constexpr int NDC = DP / 16;
-  const int lane = threadIdx.x, l32 = lane & 31, hh = lane >> 5;
-  const int nkb = (a.N + 63) / 64;
-  const int kt = (int)(blockIdx.x % (unsigned)nkb);
-  const int bh = (int)(blockIdx.x / (unsigned)nkb);
+template <typename E, int DP, int VEC, int KT>
+__global__ __launch_bounds__(64 * snap_waves(DP)) void snap_scores_kernel(const SnapArgs a) {
+  constexpr int NDC = DP / 16, NW = snap_waves(DP), NT = 64 * NW;
+  __shared__ u32x4 qrows[kSnapChunk * 32 * (DP / 8)];  // K on the way to registers, then Q
+  __shared__ __attribute__((aligned(16))) float st_m[kSnapLdsRows], st_il[kSnapLdsRows];
+  __shared__ float2 sm[NT];
+  __shared__ float red[NW][64];
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wv % a.KG, rp = wv / a.KG, RP = NW / a.KG;
+  const int bh = (int)(blockIdx.x % (unsigned)a.BH), blk = (int)(blockIdx.x / (unsigned)a.BH);
   const int b = bh / a.Hkv, hkv = bh - b * a.Hkv;
-  const int kb = kt * 64;
+  const int kb = (blk * a.KG + kg) * 32 * KT;
   const u16* kbase = a.k + b * a.ks[0] + hkv * a.ks[1];
 
-  // K fragments (B operand) of the block's 64 keys, loaded once for every row tile
-  u32x4 kf[2][NDC];
+  u32x4 kf[KT][NDC];                              // K fragments (B operand) of the wave's keys
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const int key = kb + 32 * s + l32;
-    const bool kok = key < a.N;
-    const u16* krow = kbase + (long long)(kok ? key : 0) * a.ks[2];
-#pragma unroll
-    for (int c = 0; c < NDC; ++c)
-      kf[s][c] = kok ? load8(krow, a.ks[3], 16 * c + 8 * hh, a.D, VEC) : (u32x4){0u, 0u, 0u, 0u};
-  }
-  float acc[2] = {0.f, 0.f};
-  for (int rt = 0; rt < a.RT; ++rt) {
-    // this lane's query row (A operand) and its statistics
-    const int r = rt * 32 + l32;
-    const bool row_ok = r < a.R;
-    int head = 0, qpos = -1;
-    if (row_ok) snap_row(a, hkv, r, head, qpos);
-    // rows with no work in this key block: every key of the block is past their position
-    if (__all(!row_ok || qpos < kb)) continue;
-    const u16* qrow = a.q + b * a.qs[0] + head * a.qs[1] + (long long)(row_ok ? qpos : 0) * a.qs[2];
-    u32x4 qf[NDC];
-#pragma unroll
-    for (int c = 0; c < NDC; ++c)
-      qf[c] = row_ok ? load8(qrow, a.qs[3], 16 * c + 8 * hh, a.D, VEC) : (u32x4){0u, 0u, 0u, 0u};
-    const float2 st = a.stats[(long long)(bh * a.RT + rt) * 32 + l32];
-    // statistics of the 16 rows a lane holds in the accumulator: 8(i/4) + 4h + i%4
-    float m_r[16], il_r[16];
-    int qp_r[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int ri = 8 * (i >> 2) + 4 * hh + (i & 3);
-      m_r[i] = __shfl(st.x, ri);
-      il_r[i] = __shfl(st.y, ri);
-      qp_r[i] = __shfl(qpos, ri);
-    }
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int key = kb + 32 * s + l32;
-      f32x16 sacc = (f32x16){};
-#pragma unroll
-      for (int c = 0; c < NDC; ++c) sacc = E::mfma(qf[c], kf[s][c], sacc);
-      // lanes hold key kb + 32s + l32; register i holds row 8(i/4) + 4h + i%4 of the tile
-      float sum = 0.f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float v = round_logit<E>(sacc[i]) * a.scale;
-        sum += key <= qp_r[i] ? expf(v - m_r[i]) * il_r[i] : 0.f;
+  for (int s = 0; s < KT; ++s)
+    snap_load_keys<DP, VEC>(a, kbase, kb + 32 * s, qrows + wv * 32 * (DP / 8), kf[s]);
+  const bool masked = kb + 32 * KT > a.N - a.W;
+  // (max, 1/sum) of row r of the chunk; padding rows of the last tile contribute nothing
+  auto put = [&](int r, float m, float il) {
+    const bool live = r < a.R;
+    st_m[r % kSnapLdsRows] = live ? m : 0.f;
+    st_il[r % kSnapLdsRows] = live ? il : 0.f;
+  };
+  float acc[KT] = {};
+  for (int r0 = 0; r0 < a.Rp; r0 += kSnapLdsRows) {
+    // statistics of rows r0 .. r0 + rows - 1 into LDS
+    const int rows = min(kSnapLdsRows, a.Rp - r0);
+    if (a.stats) {
+      if (r0 > 0) __syncthreads();
+      for (int r = tid; r < rows; r += NT) {
+        const float2 v = a.stats[(long long)bh * a.Rp + r0 + r];
+        put(r0 + r, v.x, v.y);
       }
-      acc[s] += sum;
+    } else {
+      // Rp <= kSnapLdsRows: few rows share the block's threads, each taking every P-th partial
+      int P = 1;
+      while (P < 8 && 2 * P * rows <= NT) P *= 2;
+      for (int i = tid; i < P * rows; i += NT) {
+        const int r = i % rows, part = i / rows;
+        float m, l;
+        snap_merge_parts(a, bh, r, part, P, m, l);
+        if (P > 1)
+          sm[i] = make_float2(m, l);
+        else
+          put(r, m, 1.f / l);
+      }
+      if (P > 1) {
+        __syncthreads();
+        if (tid < rows) {
+          float m = sm[tid].x, l = sm[tid].y;
+          for (int p = 1; p < P; ++p) snap_merge(a, m, l, sm[p * rows + tid].x, sm[p * rows + tid].y);
+          put(tid, m, 1.f / l);
+        }
+      }
+    }
+    for (int rt0 = r0 / 32; rt0 < (r0 + rows) / 32; rt0 += kSnapChunk) {
+    __syncthreads();                             // the buffer's last readers are done
+    snap_load_rows<DP, VEC, NT>(a, b, hkv, rt0, qrows);
+    __syncthreads();
+    for (int rt = rt0 + rp; rt < min(rt0 + kSnapChunk, a.RT); rt += RP) {
+      f32x16 x[KT];
+#pragma unroll
+      for (int c = 0; c < NDC; ++c) {
+        const u32x4 qf = snap_frag<DP>(qrows, (rt - rt0) * 32 + l32, 2 * c + hh);
+#pragma unroll
+        for (int s = 0; s < KT; ++s)
+          x[s] = c == 0 ? E::mfma(qf, kf[s][0], (f32x16){}) : E::mfma(qf, kf[s][c], x[s]);
+      }
+      const int qpos = masked ? snap_qpos(a, rt * 32 + l32) : 0;
+#pragma unroll
+      for (int s = 0; s < KT; ++s) round_logits<E>(x[s]);
+      // lanes hold key kb + 32s + l32; register i holds row 8(i/4) + 4h + i%4 of the tile
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int rj = rt * 32 - r0 + 8 * j + 4 * hh;
+        const float4 m4 = *(const float4*)(st_m + rj), il4 = *(const float4*)(st_il + rj);
+        const float mr[4] = {m4.x, m4.y, m4.z, m4.w}, ilr[4] = {il4.x, il4.y, il4.z, il4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int qp = masked ? __shfl(qpos, 8 * j + 4 * hh + e) : 0;
+#pragma unroll
+          for (int s = 0; s < KT; ++s) {
+            const float p = snap_exp(a, x[s][4 * j + e] - mr[e]) * ilr[e];
+            acc[s] += !masked || kb + 32 * s + l32 <= qp ? p : 0.f;
+          }
+        }
+      }
+    }
     }
   }
-  // lanes h = 0 and 1 hold the two halves of the rows of each key; lane l of half s stores
-  // key kb + 32s + l32
-  const float t0 = half_swap_sum(acc[0]), t1 = half_swap_sum(acc[1]);
+  // lanes h = 0 and 1 hold the two halves of the rows of each key, the row parts' waves the
+  // other row tiles; lane l of half s holds key kb + 32s + l32
+  const float t0 = half_swap_sum(acc[0]), t1 = half_swap_sum(acc[KT - 1]);
+  red[wv][lane] = hh == 0 ? t0 : t1;
+  __syncthreads();
   const int key = kb + 32 * hh + l32;
-  if (key < a.N) a.scores[(long long)bh * a.N + key] = (hh == 0 ? t0 : t1) / (float)a.G;
+  if (rp == 0 && hh < KT && key < a.N) {
+    float t = red[kg][lane];
+    for (int p = 1; p < RP; ++p) t += red[p * a.KG + kg][lane];
+    a.scores[(long long)bh * a.N + key] = t / (float)a.G;
+  }
 }
 
 struct SnapKernel {
@@ -210,22 +365,24 @@ struct SnapKernel {
   const char* name;
 };
 
-// Index (dtype, DP, VEC) -> 2 * (4 * dtype + 2 * dpi + vec) (+1 for the scores kernel);
-// VEC = 1: 16-byte row loads (channel stride 1, 16-byte aligned rows), 0: element loads.
-#define FE_SNAP_KERNELS(E, DP, V, TAG)                                                            \
-  {(const void*)snap_stats_kernel<E, DP, V>, "snap_stats_kernel<" TAG "," #DP "," #V ">"},         \
-      {(const void*)snap_scores_kernel<E, DP, V>, "snap_scores_kernel<" TAG "," #DP "," #V ">"}
+// Index ((dtype * 3 + tile dim 64, 128, 256) * 2 + VEC) * 4 + 2 * (KT - 1) (+1 for the scores
+// kernel); VEC = 1: 16-byte row loads (channel stride 1, 16-byte aligned rows), 0: element loads.
+#define FE_SNAP_KT(E, DP, V, KT, TAG)                                                                       \
+  {(const void*)snap_stats_kernel<E, DP, V, KT>, "snap_stats_kernel<" TAG "," #DP "," #V "," #KT ">"},       \
+      {(const void*)snap_scores_kernel<E, DP, V, KT>, "snap_scores_kernel<" TAG "," #DP "," #V "," #KT ">"}
+#define FE_SNAP_VEC(E, DP, V, TAG) FE_SNAP_KT(E, DP, V, 1, TAG), FE_SNAP_KT(E, DP, V, 2, TAG)
+#define FE_SNAP_DIM(E, DP, TAG) FE_SNAP_VEC(E, DP, 0, TAG), FE_SNAP_VEC(E, DP, 1, TAG)
+#define FE_SNAP_TYPE(E, TAG) FE_SNAP_DIM(E, 64, TAG), FE_SNAP_DIM(E, 128, TAG), FE_SNAP_DIM(E, 256, TAG)
 
 const SnapKernel kSnapKernels[] = {
-    FE_SNAP_KERNELS(F16, 64, 0, "f16"),   FE_SNAP_KERNELS(F16, 64, 1, "f16"),
-    FE_SNAP_KERNELS(F16, 128, 0, "f16"),  FE_SNAP_KERNELS(F16, 128, 1, "f16"),
-    FE_SNAP_KERNELS(BF16, 64, 0, "bf16"), FE_SNAP_KERNELS(BF16, 64, 1, "bf16"),
-    FE_SNAP_KERNELS(BF16, 128, 0, "bf16"), FE_SNAP_KERNELS(BF16, 128, 1, "bf16"),
-    FE_SNAP_KERNELS(F16, 256, 0, "f16"),  FE_SNAP_KERNELS(F16, 256, 1, "f16"),
-    FE_SNAP_KERNELS(BF16, 256, 0, "bf16"), FE_SNAP_KERNELS(BF16, 256, 1, "bf16"),
+    FE_SNAP_TYPE(F16, "f16"),
+    FE_SNAP_TYPE(BF16, "bf16"),
     {(const void*)snap_combine_kernel, "snap_combine_kernel"},
 };
-#undef FE_SNAP_KERNELS
+#undef FE_SNAP_TYPE
+#undef FE_SNAP_DIM
+#undef FE_SNAP_VEC
+#undef FE_SNAP_KT
 
 void append_snap_resources(std::string& out) {
   for (const auto& e : kSnapKernels) {
@@ -241,14 +398,16 @@ void append_snap_resources(std::string& out) {
   }
 }
 
-// Key splits of the statistics pass: enough waves to cover the chip (about 2048), at
-// least one 64-key tile per split.
-void snap_split(long long BH, long long RT, long long ntiles, int& S, int& per) {
-  long long s = (2048 + BH * RT - 1) / (BH * RT);
-  if (s < 1) s = 1;
-  if (s > ntiles) s = ntiles;
-  per = (int)((ntiles + s - 1) / s);
-  S = (int)((ntiles + per - 1) / per);
+// Key blocks: KG groups of KT 32-key halves each. The largest block (512 keys, each K fragment in
+// registers serving every row tile) that still gives every CU one; short prompts take fewer keys
+// per block and give the waves different row tiles instead. Blocks per (b, kv head): the result.
+int snap_split(long long BH, long long N, int waves, int& KG, int& KT) {
+  KG = waves;
+  KT = 2;
+  auto blocks = [&]() { return (N + 32 * KG * KT - 1) / (32 * KG * KT); };
+  while (KG > 1 && BH * blocks() < 256) KG /= 2;
+  if (KG == 1 && BH * blocks() < 256) KT = 1;
+  return (int)blocks();
 }
 
 bool snap_vec(const void* p, const int64_t* st, int64_t D) {
@@ -263,9 +422,9 @@ using namespace fe;
 extern "C" size_t fe_snap_scores_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t N, int64_t window) {
   if (B < 1 || Hq < 1 || Hkv < 1 || N < 1 || window < 1 || Hq % Hkv != 0) return 0;
   const long long W = window < N ? window : N;
-  const long long BH = B * Hkv, R = (Hq / Hkv) * W, RT = (R + 31) / 32, ntiles = (N + 63) / 64;
-  int S, per;
-  snap_split(BH, RT, ntiles, S, per);
+  const long long BH = B * Hkv, R = (Hq / Hkv) * W, RT = (R + 31) / 32;
+  int KG, KT;
+  const int S = snap_split(BH, N, snap_waves(256), KG, KT);   // the most blocks of any head dim
   return (size_t)(BH * RT * 32) * sizeof(float2) * (size_t)(S + 1);
 }
 
@@ -295,17 +454,13 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
       return FE_ERR_INVALID;
     }
   const long long W = window < N ? window : N;
-  const long long G = Hq / Hkv, BH = B * Hkv, R = G * W, RT = (R + 31) / 32, ntiles = (N + 63) / 64;
-  if (N > (1LL << 30) || R > (1LL << 30) || BH * RT * 32 > (1LL << 40) || BH * ntiles > 0x7fffffffLL) {
+  const long long G = Hq / Hkv, BH = B * Hkv, R = G * W, RT = (R + 31) / 32;
+  if (N > (1LL << 30) || R > (1LL << 30) || BH * RT * 32 > (1LL << 40) || BH * ((N + 31) / 32) > 0x7fffffffLL) {
     set_error("fe_snap_scores: problem too large");
     return FE_ERR_UNSUPPORTED;
   }
-  int S, per;
-  snap_split(BH, RT, ntiles, S, per);
-  if (BH * RT * S > 0x7fffffffLL) {
-    set_error("fe_snap_scores: problem too large");
-    return FE_ERR_UNSUPPORTED;
-  }
+  int KG, KT;
+  const int waves = snap_waves(D <= 128 ? 128 : 256), S = snap_split(BH, N, waves, KG, KT);
   const size_t need = fe_snap_scores_workspace_bytes(B, Hq, Hkv, N, window);
   if (!workspace || workspace_bytes < need) {
     set_error("fe_snap_scores: needs a workspace of fe_snap_scores_workspace_bytes() bytes");
@@ -316,7 +471,7 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
   a.k = (const u16*)k;
   a.scores = scores;
   a.part = (float2*)workspace;
-  a.stats = a.part + BH * RT * 32 * S;
+  a.stats = RT * 32 > kSnapLdsRows ? a.part + BH * RT * 32 * S : nullptr;
   for (int i = 0; i < 4; ++i) {
     a.qs[i] = q_strides[i];
     a.ks[i] = k_strides[i];
@@ -329,25 +484,25 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
   a.W = (int)W;
   a.R = (int)R;
   a.RT = (int)RT;
+  a.Rp = (int)(RT * 32);
   a.S = S;
-  a.tiles_per_split = per;
-  a.ntiles = (int)ntiles;
-  a.scale = (float)pow((double)D, -0.5);
+  a.KG = KG;
+  a.scale_log2 = (float)(1.4426950408889634 * pow((double)D, -0.5));
   const int vec = snap_vec(q, q_strides, D) && snap_vec(k, k_strides, D) ? 1 : 0;
   const int bf = dtype == FE_DTYPE_BF16 ? 1 : 0;
-  const int ki = D <= 128 ? 4 * bf + 2 * (D <= 64 ? 0 : 1) + vec : 8 + 2 * bf + vec;
-  const void* stats_fn = kSnapKernels[2 * ki].fn;
-  const void* scores_fn = kSnapKernels[2 * ki + 1].fn;
+  const int ki = ((bf * 3 + (D <= 64 ? 0 : (D <= 128 ? 1 : 2))) * 2 + vec) * 4 + 2 * (KT - 1);
+  const void* stats_fn = kSnapKernels[ki].fn;
+  const void* scores_fn = kSnapKernels[ki + 1].fn;
   hipStream_t stream = (hipStream_t)hip_stream;
   void* kargs[] = {&a};
-  hipError_t err = hipLaunchKernel(stats_fn, dim3((unsigned)(BH * RT * S)), dim3(64), kargs, 0, stream);
-  if (err == hipSuccess) {
+  const dim3 grid((unsigned)(BH * S)), block(64 * waves);
+  hipError_t err = hipLaunchKernel(stats_fn, grid, block, kargs, 0, stream);
+  if (err == hipSuccess && a.stats) {
     const long long rows = BH * RT * 32;
     err = hipLaunchKernel((const void*)snap_combine_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), kargs,
                           0, stream);
   }
-  if (err == hipSuccess)
-    err = hipLaunchKernel(scores_fn, dim3((unsigned)(BH * ntiles)), dim3(64), kargs, 0, stream);
+  if (err == hipSuccess) err = hipLaunchKernel(scores_fn, grid, block, kargs, 0, stream);
   if (err != hipSuccess) {
     set_error(std::string("fe_snap_scores: launch: ") + hipGetErrorString(err));
     return FE_ERR_HIP;
