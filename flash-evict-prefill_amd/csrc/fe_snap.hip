@@ -22,8 +22,8 @@
 // What bounds it: K is read once from HBM (33.5 MB at N = 32768, 4 KV heads: 7 us) and each
 // logit takes two exponentials (2 x 29 M at 28 heads x 32 rows, 10 us of vector work); launches
 // and the latency of each step make the rest. Layout: a wave keeps the K fragments of its keys in
-// registers and runs over the row tiles, whose Q fragments it reads one tile ahead. (One row tile
-// per wave against a strip of K, 64-thread blocks, read K once per row tile and left a combine
+// registers and runs over the row tiles, whose Q the block holds in LDS, eight tiles at a time. (One
+// row tile per wave against a strip of K, 64-thread blocks, read K once per row tile and left a combine
 // kernel of few threads with a serial loop over the strips: 47.6 + 37.2 + 35.0 us at 28/4 heads,
 // N = 32768, D = 128, window 32, against 19.0 + 23.6 us here.)
 #include <math.h>
@@ -46,7 +46,7 @@ struct SnapArgs {
   const u16* k;
   float* scores;
   float2* part;          // [BH][S][Rp] (max, sum) partials
-  float2* stats;         // [BH][Rp] (max, 1/sum), windows of more than kSnapLdsRows rows
+  float2* stats;         // [BH][Rp] (max, sum), windows of more than kSnapLdsRows rows
   long long qs[4], ks[4];
   int N, D, G, Hkv, BH;
   int W, R, RT, Rp;      // window rows per head, rows per group (G*W), 32-row tiles, 32 * RT
@@ -222,8 +222,8 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_stats_kernel(const S
   }
 }
 
-// (max, 1/sum) of row r of a group from partials s0, s0 + step, ... of its key blocks; four loads
-// in flight. Every row of the window sees at least key 0.
+// (max, sum) of row r of a group from partials s0, s0 + step, ... of its key blocks; four loads
+// in flight.
 __device__ __forceinline__ void snap_merge_parts(const SnapArgs& a, int bh, int r, int s0, int step, float& m, float& l) {
   const float2* p = a.part + (long long)bh * a.S * a.Rp + r;
   m = -__builtin_huge_valf();
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(256) void snap_combine_kernel(const SnapArgs a) {
   const int bh = (int)(i / a.Rp), r = (int)(i - (long long)bh * a.Rp);
   float m, l;
   snap_merge_parts(a, bh, r, 0, 1, m, l);
-  a.stats[i] = make_float2(m, 1.f / l);
+  a.stats[i] = make_float2(m, l);
 }
 
 template <typename E, int DP, int VEC, int KT>
@@ -274,11 +274,12 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_scores_kernel(const 
   for (int s = 0; s < KT; ++s)
     snap_load_keys<DP, VEC>(a, kbase, kb + 32 * s, qrows + wv * 32 * (DP / 8), kf[s]);
   const bool masked = kb + 32 * KT > a.N - a.W;
-  // (max, 1/sum) of row r of the chunk; padding rows of the last tile contribute nothing
-  auto put = [&](int r, float m, float il) {
-    const bool live = r < a.R;
+  // max and 1/sum of row r; padding rows of the last tile, and rows whose every logit is -inf,
+  // contribute nothing
+  auto put = [&](int r, float m, float l) {
+    const bool live = r < a.R && l != 0.f;
     st_m[r % kSnapLdsRows] = live ? m : 0.f;
-    st_il[r % kSnapLdsRows] = live ? il : 0.f;
+    st_il[r % kSnapLdsRows] = live ? 1.f / l : 0.f;
   };
   float acc[KT] = {};
   for (int r0 = 0; r0 < a.Rp; r0 += kSnapLdsRows) {
@@ -301,50 +302,50 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_scores_kernel(const 
         if (P > 1)
           sm[i] = make_float2(m, l);
         else
-          put(r, m, 1.f / l);
+          put(r, m, l);
       }
       if (P > 1) {
         __syncthreads();
         if (tid < rows) {
           float m = sm[tid].x, l = sm[tid].y;
           for (int p = 1; p < P; ++p) snap_merge(a, m, l, sm[p * rows + tid].x, sm[p * rows + tid].y);
-          put(tid, m, 1.f / l);
+          put(tid, m, l);
         }
       }
     }
     for (int rt0 = r0 / 32; rt0 < (r0 + rows) / 32; rt0 += kSnapChunk) {
-    __syncthreads();                             // the buffer's last readers are done
-    snap_load_rows<DP, VEC, NT>(a, b, hkv, rt0, qrows);
-    __syncthreads();
-    for (int rt = rt0 + rp; rt < min(rt0 + kSnapChunk, a.RT); rt += RP) {
-      f32x16 x[KT];
+      __syncthreads();                             // the buffer's last readers are done
+      snap_load_rows<DP, VEC, NT>(a, b, hkv, rt0, qrows);
+      __syncthreads();
+      for (int rt = rt0 + rp; rt < min(rt0 + kSnapChunk, a.RT); rt += RP) {
+        f32x16 x[KT];
 #pragma unroll
-      for (int c = 0; c < NDC; ++c) {
-        const u32x4 qf = snap_frag<DP>(qrows, (rt - rt0) * 32 + l32, 2 * c + hh);
+        for (int c = 0; c < NDC; ++c) {
+          const u32x4 qf = snap_frag<DP>(qrows, (rt - rt0) * 32 + l32, 2 * c + hh);
 #pragma unroll
-        for (int s = 0; s < KT; ++s)
-          x[s] = c == 0 ? E::mfma(qf, kf[s][0], (f32x16){}) : E::mfma(qf, kf[s][c], x[s]);
-      }
-      const int qpos = masked ? snap_qpos(a, rt * 32 + l32) : 0;
+          for (int s = 0; s < KT; ++s)
+            x[s] = c == 0 ? E::mfma(qf, kf[s][0], (f32x16){}) : E::mfma(qf, kf[s][c], x[s]);
+        }
+        const int qpos = masked ? snap_qpos(a, rt * 32 + l32) : 0;
 #pragma unroll
-      for (int s = 0; s < KT; ++s) round_logits<E>(x[s]);
-      // lanes hold key kb + 32s + l32; register i holds row 8(i/4) + 4h + i%4 of the tile
+        for (int s = 0; s < KT; ++s) round_logits<E>(x[s]);
+        // lanes hold key kb + 32s + l32; register i holds row 8(i/4) + 4h + i%4 of the tile
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int rj = rt * 32 - r0 + 8 * j + 4 * hh;
-        const float4 m4 = *(const float4*)(st_m + rj), il4 = *(const float4*)(st_il + rj);
-        const float mr[4] = {m4.x, m4.y, m4.z, m4.w}, ilr[4] = {il4.x, il4.y, il4.z, il4.w};
+        for (int j = 0; j < 4; ++j) {
+          const int rj = rt * 32 - r0 + 8 * j + 4 * hh;
+          const float4 m4 = *(const float4*)(st_m + rj), il4 = *(const float4*)(st_il + rj);
+          const float mr[4] = {m4.x, m4.y, m4.z, m4.w}, ilr[4] = {il4.x, il4.y, il4.z, il4.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int qp = masked ? __shfl(qpos, 8 * j + 4 * hh + e) : 0;
+          for (int e = 0; e < 4; ++e) {
+            const int qp = masked ? __shfl(qpos, 8 * j + 4 * hh + e) : 0;
 #pragma unroll
-          for (int s = 0; s < KT; ++s) {
-            const float p = snap_exp(a, x[s][4 * j + e] - mr[e]) * ilr[e];
-            acc[s] += !masked || kb + 32 * s + l32 <= qp ? p : 0.f;
+            for (int s = 0; s < KT; ++s) {
+              const float p = snap_exp(a, x[s][4 * j + e] - mr[e]) * ilr[e];
+              acc[s] += !masked || kb + 32 * s + l32 <= qp ? p : 0.f;
+            }
           }
         }
       }
-    }
     }
   }
   // lanes h = 0 and 1 hold the two halves of the rows of each key, the row parts' waves the

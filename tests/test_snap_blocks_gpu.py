@@ -30,3 +30,19 @@ def test_snap_block_shapes_match_oracle(b, hq, hk, n, d, w, dtype, layout):
     got = snap_scores(q, k, w)
     torch.cuda.synchronize()
     _check_scores(got, osnap.snap_scores(q.cpu(), k.cpu(), w), min(w, n))
+
+
+@pytest.mark.parametrize("w", [32, 2100])
+def test_rows_of_minus_infinity_contribute_nothing(w):
+    """fp16 products below -65504 round to -inf; a row whose every logit is -inf has no softmax and
+    adds nothing to any key (w = 2100: statistics from the combine kernel). The other head's rows
+    are unchanged by it."""
+    n, d = 2500, 128
+    q, k = _qk(1, 2, 1, n, d, torch.float16, 77)
+    k[...] = -k.abs() - 1
+    q[:, 0] = 500.0
+    got = snap_scores(q, k, w)
+    alone = snap_scores(q[:, 1:].contiguous(), k, w)
+    torch.cuda.synchronize()
+    assert torch.isfinite(got).all()
+    torch.testing.assert_close(got, alone / 2, rtol=1e-5, atol=0)
