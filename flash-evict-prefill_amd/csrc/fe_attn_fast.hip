@@ -265,6 +265,15 @@ __device__ __forceinline__ int block_item(const AttnArgs& a, int* s_item, int wv
   return __builtin_amdgcn_readfirstlane(*s_item);
 }
 
+// Word and bit of attention item i in AttnArgs::done: consecutive items on the 16 lines (of 32
+// words) in turn. The replay items of a launch wait for the heaviest items, which are numbered one
+// after the other: with all their bits in one word, some hundred workgroups polled one line, and
+// every K/V tile read from that line's memory channel queued behind them (attention items 1.7 times
+// as long: B1 Hq32/Hkv8 D64, every row replayed, N4096 214 -> 154 us a layer, N2048 112 -> 63;
+// B2 Hq12/Hkv4 D80 N1531 71 -> 52).
+__device__ __forceinline__ int done_word(int i) { return ((i & 15) << 5) | ((i >> 4) & 31); }
+__device__ __forceinline__ unsigned done_bit(int i) { return 1u << (i >> 9); }
+
 // Replay items of the attention kernels: lane 0 of the calling wave waits
 // until attention item `dep` has published its rows' replay biases (its bit in a.done) and
 // returns whether it has. The bias words are written and read as agent-scope relaxed atomics
@@ -281,8 +290,8 @@ __device__ __forceinline__ int block_item(const AttnArgs& a, int* s_item, int wv
 __device__ __forceinline__ bool wait_item_done(const AttnArgs& a, int dep, int dep_tiles) {
   bool ok = true;
   if (lane_now() == 0) {
-    const unsigned bit = 1u << (dep & 31);
-    unsigned* w = a.done + (dep >> 5);
+    const unsigned bit = done_bit(dep);
+    unsigned* w = a.done + done_word(dep);
     const int polls = a.wait_base + a.wait_per_tile * dep_tiles;
     ok = false;
     for (int spin = 0; spin < polls && !ok; ++spin) {
@@ -685,7 +694,7 @@ __global__ __launch_bounds__(NW * 64, (FastOccupancy<NW, DP>::WAVES_PER_EU)) voi
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (wv == 0 && lane_now() == 0)
-          __hip_atomic_fetch_or(a.done + (item >> 5), 1u << (item & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_fetch_or(a.done + done_word(item), done_bit(item), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       return;
     }
@@ -1307,7 +1316,7 @@ __global__ __launch_bounds__(512, 2) void attn_rt2_kernel(const AttnArgs a) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (wv == 0 && lane_now() == 0)
-        __hip_atomic_fetch_or(a.done + (item >> 5), 1u << (item & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_or(a.done + done_word(item), done_bit(item), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   };
 
