@@ -722,6 +722,9 @@ int64_t one_shot_grid(int64_t items) { return items + ((items / 8 + 7) & ~(int64
 #ifndef FE_REPLAY_ROUNDS_SPLIT
 #define FE_REPLAY_ROUNDS_SPLIT 1
 #endif
+#ifndef FE_SMALL_ITEM_MIN_TILES
+#define FE_SMALL_ITEM_MIN_TILES 2
+#endif
 #ifndef FE_REPLAY_ITEM_MIN_TILES
 #define FE_REPLAY_ITEM_MIN_TILES 8
 #endif
@@ -969,6 +972,13 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
     const int64_t rs_max = (max_tiles + FE_REPLAY_ITEM_MIN_TILES - 1) / FE_REPLAY_ITEM_MIN_TILES;
     int64_t rs = nwg > 0 ? (FE_REPLAY_ITEMS_PER_WG * resident + nwg - 1) / nwg : 1;
     rs = rs < 1 ? 1 : (rs > rs_max ? rs_max : rs);
+    // With workgroups to spare (every item in the first wave), shorter key ranges, down to
+    // FE_SMALL_ITEM_MIN_TILES key tiles: the launch ends with the replay of the heaviest rows, all of
+    // it serial after their attention items. In more items than that the rows' Q, biases and waits
+    // cost more than the shorter ranges save.
+    const int64_t free_rs = nwg > 0 ? (resident - items) / nwg : 0;
+    const int64_t short_rs = (max_tiles + FE_SMALL_ITEM_MIN_TILES - 1) / FE_SMALL_ITEM_MIN_TILES;
+    if (rs < free_rs && rs < short_rs) rs = free_rs < short_rs ? free_rs : short_rs;
     if (nwg > 0 && items + nwg * rs < (int64_t)0x7fffffff) {
       replay_items = true;
       a.nattn = (int)items;
