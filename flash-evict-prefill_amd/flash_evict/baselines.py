@@ -44,15 +44,15 @@ def snap_scores(q, k, window=32):
         raise ValueError("CUDA fp16 or bf16 inputs required")
     if isinstance(window, bool) or not isinstance(window, int) or window < 1:
         raise ValueError("window must be a positive integer")
-    scores = torch.empty((b, hk, n), dtype=torch.float32, device=q.device)
+    device = q.device
+    scores = torch.empty((b, hk, n), dtype=torch.float32, device=device)
     L = _lib.lib()
     ws_bytes = L.fe_snap_scores_workspace_bytes(b, hq, hk, n, window)
-    with torch.cuda.device(q.device):
-        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
-        stream = torch.cuda.current_stream(q.device).cuda_stream
+    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
+    with _lib.on_device(device):
         rc = L.fe_snap_scores(q.data_ptr(), k.data_ptr(), scores.data_ptr(), b, hq, hk, n, d,
                               _lib.strides(q), _lib.strides(k), _DTYPES[q.dtype], window,
-                              ws.data_ptr(), ws_bytes, stream)
+                              ws.data_ptr(), ws_bytes, _lib.current_stream(device))
     _lib.check(rc, "fe_snap_scores")
     return scores
 

@@ -30,16 +30,17 @@ def gather_tokens(cache, indices):
         raise ValueError("indices must be int64")
     if not cache.is_cuda or indices.device != cache.device:
         raise ValueError("gather_tokens needs CUDA (HIP) tensors on one device")
-    if any(s < 0 for s in cache.stride()) or any(s < 0 for s in indices.stride()):
+    if min(cache.stride()) < 0 or min(indices.stride()) < 0:
         raise ValueError("negative strides are not supported")
     k = indices.shape[2]
-    out = torch.empty((b, h, k, d), dtype=cache.dtype, device=cache.device)
+    device = cache.device
+    out = torch.empty((b, h, k, d), dtype=cache.dtype, device=device)
     if out.numel() == 0:
         return out
     L = _lib.lib()
-    with torch.cuda.device(cache.device):
-        stream = torch.cuda.current_stream(cache.device).cuda_stream
+    with _lib.on_device(device):
         rc = L.fe_gather_rows(cache.data_ptr(), indices.data_ptr(), out.data_ptr(), b, h, n, d, k,
-                              _lib.strides(cache), _lib.strides(indices), cache.element_size(), stream)
+                              _lib.strides(cache), _lib.strides(indices), cache.element_size(),
+                              _lib.current_stream(device))
     _lib.check(rc, "fe_gather_rows")
     return out

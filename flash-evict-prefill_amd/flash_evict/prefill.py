@@ -21,19 +21,20 @@ _DTYPES = {torch.float16: _lib.FE_DTYPE_F16, torch.bfloat16: _lib.FE_DTYPE_BF16}
 
 def _validate(q, k, v):
     """Reject inputs the kernel does not define (reference prefill.py:86-99)."""
-    if any(t.ndim != 4 for t in (q, k, v)):
+    if q.ndim != 4 or k.ndim != 4 or v.ndim != 4:
         raise ValueError("Q/K/V must have shape [batch, heads, tokens, channels]")
     b, h, n, d = q.shape
-    if (min(b, h, n, d, k.shape[1]) < 1 or k.shape != v.shape or k.shape[0] != b
-            or tuple(k.shape[2:]) != (n, d)):
+    kb, hk, kn, kd = ks = k.shape
+    if min(b, h, n, d, hk) < 1 or ks != v.shape or kb != b or kn != n or kd != d:
         raise ValueError("Expected nonempty self-attention Q/K/V with equal sequence and channel dimensions")
-    if h % k.shape[1] or d > 256:
+    if h % hk or d > 256:
         raise ValueError("Query heads must be divisible by KV heads; head dimension must be <= 256")
-    if any(t.device != q.device or t.dtype != q.dtype for t in (k, v)):
+    device, dtype = q.device, q.dtype
+    if k.device != device or v.device != device or k.dtype != dtype or v.dtype != dtype:
         raise ValueError("Q/K/V must have the same device and dtype")
-    if not q.is_cuda or q.dtype not in _DTYPES:
+    if not q.is_cuda or dtype not in _DTYPES:
         raise ValueError("CUDA fp16 or bf16 inputs required")
-    if torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v)):
+    if (q.requires_grad or k.requires_grad or v.requires_grad) and torch.is_grad_enabled():
         raise ValueError("Inference only: no backward implementation")
 
 
@@ -67,23 +68,23 @@ def prefill(q, k, v, *, causal=True, value_weighted=True, score=True,
         raise ValueError("scale must be finite")
     b, h, n, d = q.shape
     hk = k.shape[1]
-    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    importance = torch.empty((b, hk, n), dtype=torch.float32, device=q.device) if score else None
+    device, dtype = q.device, q.dtype
+    out = torch.empty((b, h, n, d), dtype=dtype, device=device)
+    importance = torch.empty((b, hk, n), dtype=torch.float32, device=device) if score else None
     window = min(n, observation_window or n)
+    score, causal, value_weighted = int(bool(score)), int(bool(causal)), int(bool(value_weighted))
     L = _lib.lib()
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        # workspace: replay biases (one float per query row), the work-item counters, and
-        # room to repack K/V the fast kernels cannot read in place
-        ws_bytes = L.fe_prefill_workspace_bytes_kv(b, h, hk, n, d, int(bool(score)), k.data_ptr(), _lib.strides(k),
-                                                   v.data_ptr(), _lib.strides(v))
-        ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=q.device) if ws_bytes else None
-        rc = L.fe_prefill_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+    k_ptr, v_ptr, k_st, v_st = k.data_ptr(), v.data_ptr(), _lib.strides(k), _lib.strides(v)
+    # workspace: replay biases (one float per query row), the work-item counters, and
+    # room to repack K/V the fast kernels cannot read in place
+    ws_bytes = L.fe_prefill_workspace_bytes_kv(b, h, hk, n, d, score, k_ptr, k_st, v_ptr, v_st)
+    ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=device) if ws_bytes else None
+    with _lib.on_device(device):
+        rc = L.fe_prefill_ws(q.data_ptr(), k_ptr, v_ptr, out.data_ptr(),
                              importance.data_ptr() if score else None,
-                             b, h, hk, n, d, _lib.strides(q), _lib.strides(k), _lib.strides(v),
-                             _DTYPES[q.dtype], scale, int(bool(causal)), int(bool(value_weighted)),
-                             int(bool(score)), recency_decay, window,
-                             ws.data_ptr() if ws is not None else None, ws_bytes, stream)
+                             b, h, hk, n, d, _lib.strides(q), k_st, v_st,
+                             _DTYPES[dtype], scale, causal, value_weighted, score, recency_decay, window,
+                             ws.data_ptr() if ws is not None else None, ws_bytes, _lib.current_stream(device))
     _lib.check(rc, "fe_prefill_ws")
     return out, importance
 
@@ -92,32 +93,37 @@ def _select(importance, budget, recent, pool_kernel, invert):
     n = importance.shape[-1]
     lead = tuple(importance.shape[:-1])
     rows = math.prod(lead)
-    x = importance.reshape(rows, n) if rows else importance.reshape(0, n)
-    if x.dtype != torch.float32:
-        x = x.float()
-    if x.stride(-1) != 1 or (rows > 1 and x.stride(0) < n):
-        x = x.contiguous()
-    row_stride = x.stride(0) if rows > 1 else n
-    indices = torch.empty((rows, budget), dtype=torch.int64, device=importance.device)
-    mask = torch.empty((rows, n), dtype=torch.bool, device=importance.device)
+    device = importance.device
+    indices = torch.empty((*lead, budget), dtype=torch.int64, device=device)
+    mask = torch.empty((*lead, n), dtype=torch.bool, device=device)
+    if rows == 0:
+        return indices, mask
+    x = importance
+    if x.dtype != torch.float32 or not x.is_contiguous():
+        x = x.reshape(rows, n)
+        if x.dtype != torch.float32:
+            x = x.float()
+        if x.stride(-1) != 1 or (rows > 1 and x.stride(0) < n):
+            x = x.contiguous()
+        row_stride = x.stride(0) if rows > 1 else n
+    else:
+        row_stride = n
     L = _lib.lib()
-    if rows:
-        if x.is_cuda:
-            ws_bytes = L.fe_select_workspace_bytes(rows, n, budget, recent, pool_kernel)
-            with torch.cuda.device(x.device):
-                ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
-                stream = torch.cuda.current_stream(x.device).cuda_stream
-                rc = L.fe_select(x.data_ptr(), rows, n, row_stride, budget, recent, pool_kernel,
-                                 indices.data_ptr(), mask.data_ptr(), int(invert),
-                                 ws.data_ptr(), ws_bytes, stream)
-            _lib.check(rc, "fe_select")
-        elif x.device.type == "cpu":
-            rc = L.fe_select_host(x.data_ptr(), rows, n, row_stride, budget, recent, pool_kernel,
-                                  indices.data_ptr(), mask.data_ptr(), int(invert))
-            _lib.check(rc, "fe_select_host")
-        else:
-            raise ValueError("select_tokens supports CUDA (HIP) and CPU tensors")
-    return indices.reshape(*lead, budget), mask.reshape(*lead, n)
+    if x.is_cuda:
+        ws_bytes = L.fe_select_workspace_bytes(rows, n, budget, recent, pool_kernel) if pool_kernel > 1 else 0
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
+        with _lib.on_device(device):
+            rc = L.fe_select(x.data_ptr(), rows, n, row_stride, budget, recent, pool_kernel,
+                             indices.data_ptr(), mask.data_ptr(), int(invert),
+                             ws.data_ptr() if ws is not None else None, ws_bytes, _lib.current_stream(device))
+        _lib.check(rc, "fe_select")
+    elif device.type == "cpu":
+        rc = L.fe_select_host(x.data_ptr(), rows, n, row_stride, budget, recent, pool_kernel,
+                              indices.data_ptr(), mask.data_ptr(), int(invert))
+        _lib.check(rc, "fe_select_host")
+    else:
+        raise ValueError("select_tokens supports CUDA (HIP) and CPU tensors")
+    return indices, mask
 
 
 def _check_selection(n, budget, recent, reserved_recent, pool_kernel):
