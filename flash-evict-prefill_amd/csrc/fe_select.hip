@@ -366,28 +366,6 @@ __device__ __forceinline__ void bracket_ranks(int K, int m, int& k_hi, int& k_lo
   has_lo = k_lo <= kSamples;
 }
 
-// f[e] for a per-lane index e without indexing the register array (which would place it in
-// scratch memory): a four-level select tree.
-__device__ __forceinline__ float pick16(const float (&f)[16], int e) {
-  // all-ones masks from the bits of e, opaque to the compiler so that the selects are not
-  // folded back into an indexed access
-  u32 m[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    m[k] = 0u - (((u32)e >> k) & 1u);
-    asm volatile("" : "+v"(m[k]));
-  }
-  auto sel = [](u32 mk, float hi, float lo) {
-    return __uint_as_float((__float_as_uint(hi) & mk) | (__float_as_uint(lo) & ~mk));
-  };
-  float a[8], b[4];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) a[j] = sel(m[0], f[2 * j + 1], f[2 * j]);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) b[j] = sel(m[1], a[2 * j + 1], a[2 * j]);
-  return sel(m[3], sel(m[2], b[3], b[2]), sel(m[2], b[1], b[0]));
-}
-
 // Eight consecutive mask bytes at p (one 8-byte store when aligned and whole).
 __device__ __forceinline__ void store_mask8(unsigned char* p, const bool (&keep)[8], int valid,
                                             unsigned char keep_v, unsigned char drop_v) {
@@ -677,16 +655,18 @@ __global__ __launch_bounds__(kSelThreads) void select_sample_kernel(const float*
     // the loop, and a fetch past the end of the row rereads its first keys (a valid
     // address), which are then ignored.
     int n_keep = 0;                               // this thread's kept keys
-    // Classification by float compares against the bracket: kept iff key > key_hi, i.e.
-    // v >= g_hi with g_hi = key_float(key_hi + 1), or v NaN while the bracket is bounded
-    // above; candidate iff key_lo <= key <= key_hi, i.e. v >= g_lo and not kept, or v NaN
-    // with the bracket open above (NaN's key is the largest).
-    bool nan_kept = false;
+    // Classification by two float compares against the bracket: kept iff key > key_hi, i.e.
+    // not v < g_hi with g_hi = key_float(key_hi + 1); candidate iff key >= key_lo, i.e. not
+    // v < g_lo, and not kept. NaN, the largest key, fails both compares, so it is kept with the
+    // bracket bounded above; open above (hi_mask 0) nothing is kept and NaN is a candidate. Bracket
+    // ends past the key of +inf have no float: the upper one opens the bracket, the lower one
+    // moves down to +inf (more candidates, the same result).
+    u32 hi_mask = 0u;
     float g_hi = 0.f, g_lo = 0.f;
     auto thresholds = [&]() __attribute__((always_inline)) {
-      nan_kept = key_hi != 0xffffffffu;
-      g_hi = nan_kept ? key_float(key_hi + 1u) : __builtin_nanf("");
-      g_lo = key_lo <= 0x007fffffu ? -__builtin_huge_valf() : key_float(key_lo);
+      hi_mask = key_hi < 0xff800000u ? 0xffffu : 0u;
+      g_hi = hi_mask ? key_float(key_hi + 1u) : 0.f;
+      g_lo = key_lo <= 0x007fffffu ? -__builtin_huge_valf() : key_float(min(key_lo, 0xff800000u));
     };
     constexpr int STEP = ST * CH;
     auto classify_row = [&](auto aligned) __attribute__((always_inline)) {
@@ -717,15 +697,15 @@ __global__ __launch_bounds__(kSelThreads) void select_sample_kernel(const float*
         }
         fetch(b, c0 + 2 * STEP);
         // bit e of kept / cand: key i0 + e is above / inside the bracket
+        // (shifted in from the top: one compare and one add with carry per bit)
         u32 kept = 0u, cand = 0u;
 #pragma unroll
-        for (int e = 0; e < CH; ++e) {
-          const float v = f[e];
-          const bool nan = v != v;
-          const bool ge_hi = v >= g_hi;
-          kept |= ((nan && nan_kept) || ge_hi ? 1u : 0u) << e;
-          cand |= ((nan && !nan_kept) || (v >= g_lo && !ge_hi) ? 1u : 0u) << e;
+        for (int e = CH - 1; e >= 0; --e) {
+          kept = kept + kept + (!(f[e] < g_hi) ? 1u : 0u);
+          cand = cand + cand + (!(f[e] < g_lo) ? 1u : 0u);
         }
+        kept &= hi_mask;
+        cand &= ~kept;
         const int nv = m - i0;                 // keys of this chunk inside the row
         const u32 vmask = nv >= CH ? 0xffffu : (nv > 0 ? (1u << nv) - 1u : 0u);
         kept &= vmask;
@@ -742,13 +722,7 @@ __global__ __launch_bounds__(kSelThreads) void select_sample_kernel(const float*
           // a lane holds few candidates: visit its set bits only
           for (u32 c = cand; c != 0u; c &= c - 1u, ++pc) {
             const int e = __builtin_ctz(c);
-            if (pc < kCandMax) {
-              const u32 ck = order_key(pick16(f, e));
-              ckey[pc] = ck;
-              c_lo = min(c_lo, ck);
-              c_hi = max(c_hi, ck);
-              cidx[pc] = i0 + e;
-            }
+            if (pc < kCandMax) cidx[pc] = i0 + e;
           }
         }
         if (mrow) {
@@ -785,6 +759,27 @@ __global__ __launch_bounds__(kSelThreads) void select_sample_kernel(const float*
       classify_row(std::false_type{});
     // full barrier: the pass's mask stores must be complete before candidates rewrite bytes
     __syncthreads();
+    n_cand = n_cand_lds;
+    // the candidates' keys, read again from the row (in L2 by now): taken out of the classifying
+    // pass's registers instead, each cost a select tree over the lane's 16 keys
+    for (int j0 = tid; j0 < min(n_cand, kCandMax); j0 += 4 * ST) {
+      float v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int j = j0 + u * ST;
+        v[u] = x[j < min(n_cand, kCandMax) ? cidx[j] : 0];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int j = j0 + u * ST;
+        if (j < min(n_cand, kCandMax)) {
+          const u32 ck = order_key(v[u]);
+          ckey[j] = ck;
+          c_lo = min(c_lo, ck);
+          c_hi = max(c_hi, ck);
+        }
+      }
+    }
     {
       // kept count, and the range of the candidate keys: the radix select below skips the
       // digits all candidates share (with the bracket open above, the bracket's own ends
@@ -807,7 +802,6 @@ __global__ __launch_bounds__(kSelThreads) void select_sample_kernel(const float*
       }
       lds_barrier();
     }
-    n_cand = n_cand_lds;
     bracketed = n_def <= K && n_def + n_cand >= K && n_cand <= kCandMax;
   }
 
