@@ -597,8 +597,9 @@ __global__ __launch_bounds__(kSelThreads) void select_sample_kernel(const float*
   static_assert(kBitRowMax / 32 >= kSamples, "the bitmap's LDS also holds the sample");
   __shared__ u32 work[kBitRowMax / 32];        // the sample, then the bitmap of kept keys
   __shared__ u32 hist[2 * 2048];
-  __shared__ u32 ckey[kCandMax];               // candidate keys
-  __shared__ int cidx[kCandMax];               // candidate indices
+  __shared__ u32 pool[2 * kCandMax];           // candidate keys, then candidate indices; at the end kept indices
+  u32* const ckey = pool;
+  int* const cidx = (int*)pool + kCandMax;
   __shared__ __attribute__((aligned(16))) int scan_tmp[2 * kSelWaves];
   __shared__ SelShared sh;
   __shared__ BracketShared bsh;
@@ -873,14 +874,27 @@ __global__ __launch_bounds__(kSelThreads) void select_sample_kernel(const float*
       for (int w = w0; w < w1; ++w) cnt += __builtin_popcount(word(w));
       int total;
       int pos = block_exclusive_scan(cnt, scan_tmp, total);
+      // Up to 2 kCandMax indices go through the candidates' LDS (free behind the scan's barriers) and
+      // out as whole lines: stored by the threads that find them, the 64 lanes of a wave write 64
+      // lines at a time.
+      const bool staged = K <= 2 * kCandMax;
       for (int w = w0; w < w1; ++w) {
         u32 v = word(w);
         while (v) {
           const int bit = __builtin_ctz(v);
-          if (pos < K) irow[pos] = 32 * w + bit;
+          if (pos < K) {
+            if (staged)
+              pool[pos] = (u32)(32 * w + bit);
+            else
+              irow[pos] = 32 * w + bit;
+          }
           ++pos;
           v &= v - 1u;
         }
+      }
+      if (staged) {
+        lds_barrier();
+        for (int j = tid; j < K; j += ST) irow[j] = (long long)pool[j];
       }
     }
   }
