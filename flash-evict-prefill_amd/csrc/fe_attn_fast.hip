@@ -325,6 +325,7 @@ __global__ __launch_bounds__(NW * 64, (FastOccupancy<NW, DP>::WAVES_PER_EU)) voi
   // above it, where two double-buffered pairs of K and V tiles would not fit the LDS, and in
   // the small-grid kernel (32 KiB of LDS per workgroup at tile dim 64: four per CU)
   constexpr int SLOTS = (DP <= 128 && !FastOccupancy<NW, DP>::SMALL_GRID) ? 2 : 1;
+  constexpr bool PIPE = FastOccupancy<NW, DP>::SMALL_GRID && DP > 64;   // tile loop: pipe_loop
   static_assert(NDC % KH == 0, "K fragment groups");
   static_assert(NW % 2 == 0 && NW >= 4, "row tiles per workgroup");
   constexpr float NEG_INF = -__builtin_huge_valf();
@@ -614,7 +615,7 @@ __global__ __launch_bounds__(NW * 64, (FastOccupancy<NW, DP>::WAVES_PER_EU)) voi
       }
     };
 
-    if (dmaw) {
+    if (!PIPE && dmaw) {
   #pragma unroll
       for (int sl = 0; sl < SLOTS; ++sl)
         if (sl < ntiles) {
@@ -622,10 +623,161 @@ __global__ __launch_bounds__(NW * 64, (FastOccupancy<NW, DP>::WAVES_PER_EU)) voi
           dma_v(sl * BN, lds_v0 + sl * TILE);
         }
     }
+
+    // Small grids at tile dims 96 and 128: the tile loop as a software pipeline within the wave, since
+    // there is at most one other wave per SIMD to fill its waits. Step t runs S(t+1) = K(t+1) Q^T one
+    // 16-channel group at a time, each followed by a share of tile t's exponentials (a wave issues in
+    // order, so vector work overlaps the matrix pipe only where it stands between two MFMAs), with
+    // the K fragments two groups ahead and the first V^T fragments read before both. K runs one tile
+    // ahead of V: K(t+1) and V(t) are read while the DMA fills K(t+2) and V(t+1), one barrier per
+    // tile. The arithmetic of every element and the order of every sum are those of t1_step.
+    // Measured, attention alone / with every row replayed, us: B1 Hq8/Hkv2 D128 N4000 79.3 / 105.8 ->
+    // 71.3 / 97.0 (one wave per SIMD; non-causal 84.6 / 130.9 -> 79.1 / 125.9), B2 the same 104.7 /
+    // 138.5 -> 98.9 / 134.8 (two). At tile dim 64 S twice needs more than the 128 registers of four
+    // waves per SIMD: at three, with spills, 7-13% slower, at two within 2%, so it keeps t1_step.
+    auto pipe_qk0 = [&](f32x16(&S)[2]) __attribute__((always_inline)) {
+  #pragma unroll
+      for (int c = 0; c < NDC; ++c)
+  #pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const u32x4 kf = *(const u32x4*)(lds_k0 + s * 1024 + koff + c * 2048);
+          S[s] = c == 0 ? E::mfma(kf, qf[0], (f32x16){}) : E::mfma(kf, qf[c], S[s]);
+        }
+    };
+    auto pipe_mask = [&](int it, f32x16(&S)[2]) __attribute__((always_inline)) {
+      const int kb = it * BN;
+      if (kb + BN - 1 > lo_lim) {
+        const int rel = qlim - kb - 4 * hh;
+  #pragma unroll
+        for (int s = 0; s < 2; ++s)
+  #pragma unroll
+          for (int i = 0; i < 16; ++i) S[s][i] = 32 * s + 8 * (i >> 2) + (i & 3) <= rel ? S[s][i] : NEG_INF;
+      }
+    };
+    // P of tile t from S (kept), and S(t+1) into SN (of whatever the buffer holds after the last tile)
+    auto pipe_main = [&](auto exact_tag, const f32x16(&S)[2], f32x16(&SN)[2], const unsigned char* kt,
+                         u32x4(&pb)[4], float(&pr)[4]) __attribute__((always_inline)) -> float {
+      constexpr bool EXACT = decltype(exact_tag)::value;
+      float ps[4];
+      // K fragments PD channel groups ahead of their MFMAs
+      constexpr int PD = 2;
+      u32x4 kf[PD][2];
+  #pragma unroll
+      for (int c = 0; c < PD; ++c)
+  #pragma unroll
+        for (int s = 0; s < 2; ++s) kf[c][s] = *(const u32x4*)(kt + s * 1024 + koff + c * 2048);
+  #pragma unroll
+      for (int c = 0; c < NDC; ++c) {
+  #pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          SN[s] = c == 0 ? E::mfma(kf[0][s], qf[0], (f32x16){}) : E::mfma(kf[c % PD][s], qf[c], SN[s]);
+          if (c + PD < NDC) kf[c % PD][s] = *(const u32x4*)(kt + s * 1024 + koff + (c + PD) * 2048);
+        }
+  #pragma unroll
+        for (int e = 2 * (c * 16 / NDC); e < 2 * ((c + 1) * 16 / NDC); e += 2) {
+          const int s = e >> 4, i = e & 15;
+          float p[2];
+  #pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            p[u] = fast_exp2(fmaf(S[s][i + u], a.abs_scale_log2, nm));
+            if constexpr (EXACT) ps[(i + u) & 3] = e + u < 4 ? p[u] : ps[(i + u) & 3] + p[u];
+          }
+          pb[e >> 3][(e & 7) >> 1] = E::pack2(p[0], p[1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  #pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        pr[j] = EXACT ? E::sum2(pb[0][j], ones2, 0.f) : E::sum2_0(pb[0][j], ones2);
+  #pragma unroll
+        for (int c = 1; c < 4; ++c) pr[j] = E::sum2(pb[c][j], ones2, pr[j]);
+      }
+      if constexpr (EXACT)
+        return (ps[0] + ps[1]) + (ps[2] + ps[3]);
+      else
+        return 0.f;
+    };
+    auto pipe_step = [&](auto exact_tag, int it, int BUF, f32x16(&S)[2], f32x16(&SN)[2])
+                         __attribute__((always_inline)) {
+      constexpr bool EXACT = decltype(exact_tag)::value;
+      if (it > 0) pipe_mask(it, S);
+      // V^T fragments of the first channel tile, read before the vector work that precedes their use
+      u32x4 vf[2][4];
+  #pragma unroll
+      for (int c4 = 0; c4 < 4; ++c4) vf[0][c4] = v_frag(BUF, 0, c4, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      u32x4 pb[4];
+      float pr[4];
+      float le = pipe_main(exact_tag, S, SN, BUF == 0 ? lds_k1 : lds_k0, pb, pr);
+      const float guard = EXACT ? le : (pr[0] + pr[1]) + (pr[2] + pr[3]);
+      if (__any(guard > E::kMaxTileSum)) {
+        const float mt = exact_max(S);
+        const float mn = vmax(m_run, mt + E::kRescaleHeadroom);
+        const float corr = mn > m_run ? fast_exp2(m_run - mn) : 1.f;
+        l_run *= corr;
+        l_rnd *= corr;
+  #pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) o[dt] *= corr;
+        m_run = mn;
+        nm = mn == NEG_INF ? 0.f : -mn;
+        le = probs(exact_tag, S, pb, pr);
+      }
+      l_rnd += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+      if constexpr (EXACT) l_run += le;
+  #pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+        if (dt + 1 < NDT) {
+  #pragma unroll
+          for (int c4 = 0; c4 < 4; ++c4) vf[(dt + 1) & 1][c4] = v_frag(BUF, 0, c4, dt + 1);
+        }
+        FE_PRIO_HI();
+  #pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4) o[dt] = E::mfma(vf[dt & 1][c4], pb[c4], o[dt]);
+        FE_PRIO_LO();
+      }
+    };
+    auto pipe_loop = [&](auto exact_tag) __attribute__((always_inline)) {
+      // tiles this wave computes: a prefix of the item's (none for a padding tile)
+      const int nact = min(ntiles, wave_hi < 0 ? 0 : wave_hi / BN + 1);
+      dma_k(0, lds_k0);
+      dma_v(0, lds_v0);
+      if (ntiles > 1) dma_k(BN, lds_k1);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      auto sync = [&](int it, int BUF) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (it + 2 < ntiles) dma_k((it + 2) * BN, BUF == 0 ? lds_k0 : lds_k1);
+        if (it + 1 < ntiles) dma_v((it + 1) * BN, BUF == 0 ? lds_v1 : lds_v0);
+      };
+      int it = 0;
+      if (nact > 0) {
+        f32x16 SA[2], SB[2];
+        pipe_qk0(SA);
+        pipe_mask(0, SA);
+        m_run = exact_max(SA);
+        nm = m_run == NEG_INF ? 0.f : -m_run;
+        for (; it + 2 <= nact; it += 2) {
+          sync(it, 0);
+          pipe_step(exact_tag, it, 0, SA, SB);
+          sync(it + 1, 1);
+          pipe_step(exact_tag, it + 1, 1, SB, SA);
+        }
+        if (it < nact) {
+          sync(it, 0);
+          pipe_step(exact_tag, it, 0, SA, SB);
+          ++it;
+        }
+      }
+      for (; it < ntiles; ++it) sync(it, it & 1);
+    };
+
     // The tile loop is instantiated twice, with and without the FP32 sum of the replay rows,
     // and each wave runs one of them: the choice is made once per wave, not per tile.
     auto t1_loop = [&](auto exact_tag) __attribute__((always_inline)) {
-      if constexpr (SLOTS == 2) {
+      if constexpr (PIPE) {
+        pipe_loop(exact_tag);
+      } else if constexpr (SLOTS == 2) {
         for (int it = 0; it < ntiles; it += 4) {
           t1_sync(it, 0);
           t1_step(exact_tag, it, 0, 0);
