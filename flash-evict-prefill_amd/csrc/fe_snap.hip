@@ -15,8 +15,8 @@
 //                        then p summed over the rows in-lane (lanes hold keys), / G, one
 //                        store per key
 // Both take the same key blocks in the same order, so the second read of a block's K finds it
-// in the L2 of the XCD that read it first. A window of more than kSnapLdsRows rows per group
-// merges its partials once, in snap_combine_kernel between the two, instead of in every block.
+// in the L2 of the XCD that read it first. Many partials (long prompts of few KV heads, wide windows)
+// are merged once, in snap_combine_kernel between the two, instead of in every block.
 // No atomics: every score is written once, in a fixed summation order.
 //
 // What bounds it: K is read once from HBM (33.5 MB at N = 32768, 4 KV heads: 7 us) and each
@@ -40,13 +40,18 @@ namespace fe {
 constexpr int snap_waves(int DP) { return DP > 128 ? 4 : 8; }
 constexpr int kSnapChunk = 8;        // row tiles between two merges of the key groups' partials
 constexpr int kSnapLdsRows = 2048;   // rows per group whose statistics a scores block keeps in LDS
+// Partials of a group up to which each scores block merges them itself (128 KiB through L2 a
+// block: about the 4.6 us of another launch). More go through snap_combine_kernel: B1 Hq7/Hkv1 D64
+// N = 40831, window 128 (319 x 896 partials), scores and selection 84 us, 211 with every block
+// merging them all.
+constexpr int kSnapMergeMax = 16384;
 
 struct SnapArgs {
   const u16* q;
   const u16* k;
   float* scores;
   float2* part;          // [BH][S][Rp] (max, sum) partials
-  float2* stats;         // [BH][Rp] (max, sum), windows of more than kSnapLdsRows rows
+  float2* stats;         // [BH][Rp] (max, sum), where snap_combine_kernel runs
   long long qs[4], ks[4];
   int N, D, G, Hkv, BH;
   int W, R, RT, Rp;      // window rows per head, rows per group (G*W), 32-row tiles, 32 * RT
@@ -245,13 +250,21 @@ __device__ __forceinline__ void snap_merge_parts(const SnapArgs& a, int bh, int 
   }
 }
 
-__global__ __launch_bounds__(256) void snap_combine_kernel(const SnapArgs a) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)a.BH * a.Rp) return;
-  const int bh = (int)(i / a.Rp), r = (int)(i - (long long)bh * a.Rp);
+// 32 rows per block, each by 32 threads that take every 32nd partial (B1 Hq7/Hkv1, N = 40831, window
+// 128: 319 partials of 896 rows).
+__global__ __launch_bounds__(1024) void snap_combine_kernel(const SnapArgs a) {
+  __shared__ float2 sm[32][33];
+  const int r32 = threadIdx.x & 31, part = threadIdx.x >> 5;
+  const int tiles = a.Rp / 32;
+  const int bh = (int)(blockIdx.x / (unsigned)tiles), r = (int)(blockIdx.x % (unsigned)tiles) * 32 + r32;
   float m, l;
-  snap_merge_parts(a, bh, r, 0, 1, m, l);
-  a.stats[i] = make_float2(m, l);
+  snap_merge_parts(a, bh, r, part, 32, m, l);
+  sm[part][r32] = make_float2(m, l);
+  __syncthreads();
+  if (part == 0) {
+    for (int p = 1; p < 32; ++p) snap_merge(a, m, l, sm[p][r32].x, sm[p][r32].y);
+    a.stats[(long long)bh * a.Rp + r] = make_float2(m, l);
+  }
 }
 
 template <typename E, int DP, int VEC, int KT>
@@ -472,7 +485,7 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
   a.k = (const u16*)k;
   a.scores = scores;
   a.part = (float2*)workspace;
-  a.stats = RT * 32 > kSnapLdsRows ? a.part + BH * RT * 32 * S : nullptr;
+  a.stats = RT * 32 > kSnapLdsRows || RT * 32 * S > kSnapMergeMax ? a.part + BH * RT * 32 * S : nullptr;
   for (int i = 0; i < 4; ++i) {
     a.qs[i] = q_strides[i];
     a.ks[i] = k_strides[i];
@@ -500,8 +513,7 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
   hipError_t err = hipLaunchKernel(stats_fn, grid, block, kargs, 0, stream);
   if (err == hipSuccess && a.stats) {
     const long long rows = BH * RT * 32;
-    err = hipLaunchKernel((const void*)snap_combine_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), kargs,
-                          0, stream);
+    err = hipLaunchKernel((const void*)snap_combine_kernel, dim3((unsigned)(rows / 32)), dim3(1024), kargs, 0, stream);
   }
   if (err == hipSuccess) err = hipLaunchKernel(scores_fn, grid, block, kargs, 0, stream);
   if (err != hipSuccess) {
