@@ -972,11 +972,13 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
     const int64_t rs_max = (max_tiles + FE_REPLAY_ITEM_MIN_TILES - 1) / FE_REPLAY_ITEM_MIN_TILES;
     int64_t rs = nwg > 0 ? (FE_REPLAY_ITEMS_PER_WG * resident + nwg - 1) / nwg : 1;
     rs = rs < 1 ? 1 : (rs > rs_max ? rs_max : rs);
-    // With workgroups to spare (every item in the first wave), shorter key ranges, down to
-    // FE_SMALL_ITEM_MIN_TILES key tiles: the launch ends with the replay of the heaviest rows, all of
-    // it serial after their attention items. In more items than that the rows' Q, biases and waits
-    // cost more than the shorter ranges save.
-    const int64_t free_rs = nwg > 0 ? (resident - items) / nwg : 0;
+    // With workgroups to spare, shorter key ranges, down to FE_SMALL_ITEM_MIN_TILES key tiles and up to
+    // half the resident workgroups in items: the launch ends with the replay of the heaviest rows, all
+    // of it serial after their attention items. In more items than that the rows' Q, biases and waits
+    // cost more than the shorter ranges save (1050 rows of B1 Hq4/Hkv1 D64 N3323 in 884 items instead
+    // of 238: 1.4% slower).
+    const int64_t spare = resident - items < resident / 2 ? resident - items : resident / 2;
+    const int64_t free_rs = nwg > 0 ? spare / nwg : 0;
     const int64_t short_rs = (max_tiles + FE_SMALL_ITEM_MIN_TILES - 1) / FE_SMALL_ITEM_MIN_TILES;
     if (rs < free_rs && rs < short_rs) rs = free_rs < short_rs ? free_rs : short_rs;
     if (nwg > 0 && items + nwg * rs < (int64_t)0x7fffffff) {
