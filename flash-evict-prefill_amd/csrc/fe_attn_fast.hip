@@ -325,6 +325,9 @@ __global__ __launch_bounds__(NW * 64, (FastOccupancy<NW, DP>::WAVES_PER_EU)) voi
   // above it, where two double-buffered pairs of K and V tiles would not fit the LDS, and in
   // the small-grid kernel (32 KiB of LDS per workgroup at tile dim 64: four per CU)
   constexpr int SLOTS = (DP <= 128 && !FastOccupancy<NW, DP>::SMALL_GRID) ? 2 : 1;
+  // replay items: the launch makes none for 12 waves, nor above tile dim 128, where their code beside
+  // the attention items' cost the tile loop registers
+  constexpr bool ITEMS = NW <= 8 && DP <= 128;
   constexpr bool PIPE = FastOccupancy<NW, DP>::SMALL_GRID && DP > 64;   // tile loop: pipe_loop
   static_assert(NDC % KH == 0, "K fragment groups");
   static_assert(NW % 2 == 0 && NW >= 4, "row tiles per workgroup");
@@ -832,7 +835,7 @@ __global__ __launch_bounds__(NW * 64, (FastOccupancy<NW, DP>::WAVES_PER_EU)) voi
       // replay items of this launch (agent-scope atomic store; after every wave's stores, one
       // lane sets the item's bit)
       const int qi = q0 + l32;
-      const bool items = NW <= 8 && a.nattn < a.nitems;  // the launch makes none for 12 waves
+      const bool items = ITEMS && a.nattn < a.nitems;
       if (hh == 0 && tv && qi < N) {
         const bool live = qi >= a.win_lo;
         const float bv = live ? (m_run + fast_log2(l_tot) - a.decay_log2 * (float)(qi - (N - 1))) : POS_INF;
@@ -1087,13 +1090,13 @@ __global__ __launch_bounds__(NW * 64, (FastOccupancy<NW, DP>::WAVES_PER_EU)) voi
   } else {
     const int item_end = a.queue ? a.nitems : (int)blockIdx.x + 1;
     for (int item = (int)blockIdx.x; item < item_end; item = a.queue ? next_item(a, &s_item, wv) : item_end) {
-      if constexpr (NW <= 8) {
+      if constexpr (ITEMS) {
         if (item < a.nattn)
           run_item(item);
         else
           run_replay(item - a.nattn);
       } else {
-        run_item(item);                            // no replay items (the launch does not make any)
+        run_item(item);
       }
     }
   }
