@@ -287,8 +287,7 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_scores_kernel(const 
   for (int s = 0; s < KT; ++s)
     snap_load_keys<DP, VEC>(a, kbase, kb + 32 * s, qrows + wv * 32 * (DP / 8), kf[s]);
   const bool masked = kb + 32 * KT > a.N - a.W;
-  // max and 1/sum of row r; padding rows of the last tile, and rows whose every logit is -inf,
-  // contribute nothing
+  // max and 1/sum of row r; rows whose every logit is -inf contribute nothing
   auto put = [&](int r, float m, float l) {
     const bool live = r < a.R && l != 0.f;
     st_m[r % kSnapLdsRows] = live ? m : 0.f;
@@ -339,7 +338,10 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_scores_kernel(const 
           for (int s = 0; s < KT; ++s)
             x[s] = c == 0 ? E::mfma(qf, kf[s][0], (f32x16){}) : E::mfma(qf, kf[s][c], x[s]);
         }
-        const int qpos = masked ? snap_qpos(a, rt * 32 + l32) : 0;
+        // padding rows are left out by their position: their zero query gives NaN against a key with an
+        // infinite channel, which 1/sum = 0 would not take out of the key's score
+        const bool sel = masked || (rt + 1) * 32 > a.R;
+        const int qpos = sel ? snap_qpos(a, rt * 32 + l32) : 0;
 #pragma unroll
         for (int s = 0; s < KT; ++s) round_logits<E>(x[s]);
         // lanes hold key kb + 32s + l32; register i holds row 8(i/4) + 4h + i%4 of the tile
@@ -350,11 +352,11 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_scores_kernel(const 
           const float mr[4] = {m4.x, m4.y, m4.z, m4.w}, ilr[4] = {il4.x, il4.y, il4.z, il4.w};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const int qp = masked ? __shfl(qpos, 8 * j + 4 * hh + e) : 0;
+            const int qp = sel ? __shfl(qpos, 8 * j + 4 * hh + e) : 0;
 #pragma unroll
             for (int s = 0; s < KT; ++s) {
               const float p = snap_exp(a, x[s][4 * j + e] - mr[e]) * ilr[e];
-              acc[s] += !masked || kb + 32 * s + l32 <= qp ? p : 0.f;
+              acc[s] += !sel || kb + 32 * s + l32 <= qp ? p : 0.f;
             }
           }
         }
