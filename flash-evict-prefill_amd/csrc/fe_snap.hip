@@ -153,10 +153,15 @@ __device__ __forceinline__ int snap_qpos(const SnapArgs& a, int r) {
 // sums round the other way).
 __device__ __forceinline__ float snap_exp(const SnapArgs& a, float x) { return fast_exp2(x * a.scale_log2); }
 
-// Merge of two softmax partials (a partial without a visible key: max -inf, sum 0).
+// What a partial's exponentials are taken against: its maximum, or 0 where no logit is above -inf. Then
+// the sum is 0 over -inf logits (a partial without a visible key), and NaN, which reaches the row's
+// sum through every merge, where the maximum passed over NaN logits only.
+__device__ __forceinline__ float snap_ref(float m) { return m == -__builtin_huge_valf() ? 0.f : m; }
+
+// Merge of two softmax partials.
 __device__ __forceinline__ void snap_merge(const SnapArgs& a, float& m, float& l, float m2, float l2) {
-  const float mn = fmaxf(m, m2);
-  if (mn != -__builtin_huge_valf()) l = l * snap_exp(a, m - mn) + l2 * snap_exp(a, m2 - mn);
+  const float mn = fmaxf(m, m2), ref = snap_ref(mn);
+  l = l * snap_exp(a, m - ref) + l2 * snap_exp(a, m2 - ref);
   m = mn;
 }
 
@@ -206,12 +211,11 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_stats_kernel(const S
         for (int i = 0; i < 16; ++i) m = fmaxf(m, x[s][i]);
       }
       m = half_swap_max(m);
-      if (m != NEG_INF) {
+      const float ref = snap_ref(m);
 #pragma unroll
-        for (int s = 0; s < KT; ++s) {
+      for (int s = 0; s < KT; ++s) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) l += snap_exp(a, x[s][i] - m);
-        }
+        for (int i = 0; i < 16; ++i) l += snap_exp(a, x[s][i] - ref);
       }
       l = half_swap_sum(l);
       if (hh == 0) sm[kg][(rt - rt0) * 32 + l32] = make_float2(m, l);
@@ -241,11 +245,10 @@ __device__ __forceinline__ void snap_merge_parts(const SnapArgs& a, int bh, int 
     float mn = m;
 #pragma unroll
     for (int u = 0; u < 4; ++u) mn = fmaxf(mn, v[u].x);
-    if (mn != -__builtin_huge_valf()) {
-      l *= snap_exp(a, m - mn);
+    const float ref = snap_ref(mn);
+    l *= snap_exp(a, m - ref);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) l += v[u].y * snap_exp(a, v[u].x - mn);
-    }
+    for (int u = 0; u < 4; ++u) l += v[u].y * snap_exp(a, v[u].x - ref);
     m = mn;
   }
 }

@@ -1,5 +1,5 @@
 """fe_snap_scores at keys with an infinite channel, beside padding rows (heads x window not a
-multiple of the 32-row tile)."""
+multiple of the 32-row tile), and at key blocks without one comparable logit (NaN)."""
 import pytest
 import torch
 
@@ -33,3 +33,21 @@ def test_padding_rows_add_nothing_to_a_key_with_an_infinite_channel(b, hq, hk, n
     _check_scores(got, osnap.snap_scores(q.cpu(), k.cpu(), w), w)
     _, keep = snap_select(got, n // 2, w, 1)
     assert not keep[..., masked].any()
+
+
+@pytest.mark.parametrize("b,hq,hk,n,d,w,dtype,lo,hi", [
+    (1, 8, 2, 3000, 128, 32, torch.bfloat16, 128, 1280),
+    (2, 4, 2, 9000, 64, 128, torch.float16, 64, 2048),
+    (1, 4, 1, 5000, 256, 40, torch.bfloat16, 4096, 4864),
+    (1, 16, 1, 2000, 64, 300, torch.bfloat16, 192, 1024),        # statistics merged once
+])
+def test_key_blocks_of_nan_reach_every_score(b, hq, hk, n, d, w, dtype, lo, hi):
+    """Keys lo .. hi-1 (multiples of 64) are NaN, so that some waves hold no other key: every row's
+    softmax has NaN terms, and every score is NaN, as for a single such key."""
+    print(f"snap_scores NaN blocks b={b} hq={hq} hk={hk} n={n} d={d} w={w} {dtype} {lo}:{hi}", flush=True)
+    q, k = _qk(b, hq, hk, n, d, dtype, 9100 + n + d)
+    k[:, :, lo:hi, 1] = float("nan")
+    got = snap_scores(q, k, w)
+    torch.cuda.synchronize()
+    assert torch.isnan(osnap.snap_scores(q.cpu(), k.cpu(), w)).all()
+    assert torch.isnan(got).all()
