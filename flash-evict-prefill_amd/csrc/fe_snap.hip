@@ -151,7 +151,15 @@ __device__ __forceinline__ int snap_qpos(const SnapArgs& a, int r) {
 // are as close as with expf(scale * logit - scale * max): 7.3e-7 to 3.6e-6 relative over ten shapes
 // of 2144 to 54886 keys, the two within 0.5% of each other on each (most of it is logits that FP32
 // sums round the other way).
-__device__ __forceinline__ float snap_exp(const SnapArgs& a, float x) { return fast_exp2(x * a.scale_log2); }
+__device__ __forceinline__ float snap_exponent(const SnapArgs& a, float x) { return x * a.scale_log2; }
+__device__ __forceinline__ float snap_exp(const SnapArgs& a, float x) { return fast_exp2(snap_exponent(a, x)); }
+
+// exp2 down to the smallest subnormal: v_exp_f32 returns 0 below 2^-126. Sums of exponentials, which
+// hold a term of 1, need nothing below that; the probabilities do, as keys are ranked by them.
+__device__ __forceinline__ float exp2_subnormal(float y) {
+  const bool sub = y < -126.f;
+  return fast_exp2(sub ? y + 64.f : y) * (sub ? 0x1p-64f : 1.f);
+}
 
 // What a partial's exponentials are taken against: its maximum, or 0 where no logit is above -inf. Then
 // the sum is 0 over -inf logits (a partial without a visible key), and NaN, which reaches the row's
@@ -296,87 +304,99 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_scores_kernel(const 
     st_m[r % kSnapLdsRows] = live ? m : 0.f;
     st_il[r % kSnapLdsRows] = live ? 1.f / l : 0.f;
   };
-  float acc[KT] = {};
-  for (int r0 = 0; r0 < a.Rp; r0 += kSnapLdsRows) {
-    // statistics of rows r0 .. r0 + rows - 1 into LDS
-    const int rows = min(kSnapLdsRows, a.Rp - r0);
-    if (a.stats) {
-      if (r0 > 0) __syncthreads();
-      for (int r = tid; r < rows; r += NT) {
-        const float2 v = a.stats[(long long)bh * a.Rp + r0 + r];
-        put(r0 + r, v.x, v.y);
+  // score of the wave's key 32hh + l32 (row part 0 only), times G
+  const int key = kb + 32 * hh + l32;
+  const bool store = rp == 0 && hh < KT && key < a.N;
+  auto score = [&](auto exp2_fn) __attribute__((always_inline)) {
+    float acc[KT] = {};
+    for (int r0 = 0; r0 < a.Rp; r0 += kSnapLdsRows) {
+      // statistics of rows r0 .. r0 + rows - 1 into LDS
+      const int rows = min(kSnapLdsRows, a.Rp - r0);
+      if (a.stats) {
+        if (r0 > 0) __syncthreads();
+        for (int r = tid; r < rows; r += NT) {
+          const float2 v = a.stats[(long long)bh * a.Rp + r0 + r];
+          put(r0 + r, v.x, v.y);
+        }
+      } else {
+        // Rp <= kSnapLdsRows: few rows share the block's threads, each taking every P-th partial
+        int P = 1;
+        while (P < 8 && 2 * P * rows <= NT) P *= 2;
+        for (int i = tid; i < P * rows; i += NT) {
+          const int r = i % rows, part = i / rows;
+          float m, l;
+          snap_merge_parts(a, bh, r, part, P, m, l);
+          if (P > 1)
+            sm[i] = make_float2(m, l);
+          else
+            put(r, m, l);
+        }
+        if (P > 1) {
+          __syncthreads();
+          if (tid < rows) {
+            float m = sm[tid].x, l = sm[tid].y;
+            for (int p = 1; p < P; ++p) snap_merge(a, m, l, sm[p * rows + tid].x, sm[p * rows + tid].y);
+            put(tid, m, l);
+          }
+        }
       }
-    } else {
-      // Rp <= kSnapLdsRows: few rows share the block's threads, each taking every P-th partial
-      int P = 1;
-      while (P < 8 && 2 * P * rows <= NT) P *= 2;
-      for (int i = tid; i < P * rows; i += NT) {
-        const int r = i % rows, part = i / rows;
-        float m, l;
-        snap_merge_parts(a, bh, r, part, P, m, l);
-        if (P > 1)
-          sm[i] = make_float2(m, l);
-        else
-          put(r, m, l);
-      }
-      if (P > 1) {
+      for (int rt0 = r0 / 32; rt0 < (r0 + rows) / 32; rt0 += kSnapChunk) {
+        __syncthreads();                             // the buffer's last readers are done
+        snap_load_rows<DP, VEC, NT>(a, b, hkv, rt0, qrows);
         __syncthreads();
-        if (tid < rows) {
-          float m = sm[tid].x, l = sm[tid].y;
-          for (int p = 1; p < P; ++p) snap_merge(a, m, l, sm[p * rows + tid].x, sm[p * rows + tid].y);
-          put(tid, m, l);
-        }
-      }
-    }
-    for (int rt0 = r0 / 32; rt0 < (r0 + rows) / 32; rt0 += kSnapChunk) {
-      __syncthreads();                             // the buffer's last readers are done
-      snap_load_rows<DP, VEC, NT>(a, b, hkv, rt0, qrows);
-      __syncthreads();
-      for (int rt = rt0 + rp; rt < min(rt0 + kSnapChunk, a.RT); rt += RP) {
-        f32x16 x[KT];
+        for (int rt = rt0 + rp; rt < min(rt0 + kSnapChunk, a.RT); rt += RP) {
+          f32x16 x[KT];
 #pragma unroll
-        for (int c = 0; c < NDC; ++c) {
-          const u32x4 qf = snap_frag<DP>(qrows, (rt - rt0) * 32 + l32, 2 * c + hh);
+          for (int c = 0; c < NDC; ++c) {
+            const u32x4 qf = snap_frag<DP>(qrows, (rt - rt0) * 32 + l32, 2 * c + hh);
 #pragma unroll
-          for (int s = 0; s < KT; ++s)
-            x[s] = c == 0 ? E::mfma(qf, kf[s][0], (f32x16){}) : E::mfma(qf, kf[s][c], x[s]);
-        }
-        // padding rows are left out by their position: their zero query gives NaN against a key with an
-        // infinite channel, which 1/sum = 0 would not take out of the key's score
-        const bool sel = masked || (rt + 1) * 32 > a.R;
-        const int qpos = sel ? snap_qpos(a, rt * 32 + l32) : 0;
+            for (int s = 0; s < KT; ++s)
+              x[s] = c == 0 ? E::mfma(qf, kf[s][0], (f32x16){}) : E::mfma(qf, kf[s][c], x[s]);
+          }
+          // padding rows are left out by their position: their zero query gives NaN against a key with an
+          // infinite channel, which 1/sum = 0 would not take out of the key's score
+          const bool sel = masked || (rt + 1) * 32 > a.R;
+          const int qpos = sel ? snap_qpos(a, rt * 32 + l32) : 0;
 #pragma unroll
-        for (int s = 0; s < KT; ++s) round_logits<E>(x[s]);
-        // lanes hold key kb + 32s + l32; register i holds row 8(i/4) + 4h + i%4 of the tile
+          for (int s = 0; s < KT; ++s) round_logits<E>(x[s]);
+          // lanes hold key kb + 32s + l32; register i holds row 8(i/4) + 4h + i%4 of the tile
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int rj = rt * 32 - r0 + 8 * j + 4 * hh;
-          const float4 m4 = *(const float4*)(st_m + rj), il4 = *(const float4*)(st_il + rj);
-          const float mr[4] = {m4.x, m4.y, m4.z, m4.w}, ilr[4] = {il4.x, il4.y, il4.z, il4.w};
+          for (int j = 0; j < 4; ++j) {
+            const int rj = rt * 32 - r0 + 8 * j + 4 * hh;
+            const float4 m4 = *(const float4*)(st_m + rj), il4 = *(const float4*)(st_il + rj);
+            const float mr[4] = {m4.x, m4.y, m4.z, m4.w}, ilr[4] = {il4.x, il4.y, il4.z, il4.w};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int qp = sel ? __shfl(qpos, 8 * j + 4 * hh + e) : 0;
+            for (int e = 0; e < 4; ++e) {
+              const int qp = sel ? __shfl(qpos, 8 * j + 4 * hh + e) : 0;
 #pragma unroll
-            for (int s = 0; s < KT; ++s) {
-              const float p = snap_exp(a, x[s][4 * j + e] - mr[e]) * ilr[e];
-              acc[s] += !sel || kb + 32 * s + l32 <= qp ? p : 0.f;
+              for (int s = 0; s < KT; ++s) {
+                const float p = exp2_fn(snap_exponent(a, x[s][4 * j + e] - mr[e])) * ilr[e];
+                acc[s] += !sel || kb + 32 * s + l32 <= qp ? p : 0.f;
+              }
             }
           }
         }
       }
     }
-  }
-  // lanes h = 0 and 1 hold the two halves of the rows of each key, the row parts' waves the
-  // other row tiles; lane l of half s holds key kb + 32s + l32
-  const float t0 = half_swap_sum(acc[0]), t1 = half_swap_sum(acc[KT - 1]);
-  red[wv][lane] = hh == 0 ? t0 : t1;
-  __syncthreads();
-  const int key = kb + 32 * hh + l32;
-  if (rp == 0 && hh < KT && key < a.N) {
-    float t = red[kg][lane];
-    for (int p = 1; p < RP; ++p) t += red[p * a.KG + kg][lane];
-    a.scores[(long long)bh * a.N + key] = t / (float)a.G;
-  }
+    // lanes h = 0 and 1 hold the two halves of the rows of each key, the row parts' waves the
+    // other row tiles; lane l of half s holds key kb + 32s + l32
+    const float t0 = half_swap_sum(acc[0]), t1 = half_swap_sum(acc[KT - 1]);
+    red[wv][lane] = hh == 0 ? t0 : t1;
+    __syncthreads();
+    float t = 0.f;
+    if (store) {
+      t = red[kg][lane];
+      for (int p = 1; p < RP; ++p) t += red[p * a.KG + kg][lane];
+    }
+    return t;
+  };
+  float t = score([](float y) { return fast_exp2(y); });
+  // v_exp_f32 returns 0 below 2^-126. The R terms of a sum of at least R * 2^-102 miss less than 2^-24
+  // of it by that; where a key's sum is smaller, the block runs once more with exp2_subnormal. Against
+  // the fast exponential alone 39.2 -> 40.0 us a call at 28/4 heads, N = 32768, D = 128, window 32,
+  // and 0.5-1.2% at window 128; choosing the exponential in every row tile took 3-5%.
+  if (__syncthreads_or(store && t < (float)a.R * 0x1p-102f)) t = score([](float y) { return exp2_subnormal(y); });
+  if (store) a.scores[(long long)bh * a.N + key] = t / (float)a.G;
 }
 
 struct SnapKernel {

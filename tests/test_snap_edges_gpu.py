@@ -1,5 +1,6 @@
 """fe_snap_scores at keys with an infinite channel, beside padding rows (heads x window not a
-multiple of the 32-row tile), and at key blocks without one comparable logit (NaN)."""
+multiple of the 32-row tile), at key blocks without one comparable logit (NaN), and with
+probabilities in FP32's subnormal range."""
 import pytest
 import torch
 
@@ -51,3 +52,29 @@ def test_key_blocks_of_nan_reach_every_score(b, hq, hk, n, d, w, dtype, lo, hi):
     torch.cuda.synchronize()
     assert torch.isnan(osnap.snap_scores(q.cpu(), k.cpu(), w)).all()
     assert torch.isnan(got).all()
+
+
+@pytest.mark.parametrize("hq,hk,n,d,w", [(4, 2, 700, 64, 32), (8, 1, 5000, 128, 20), (2, 1, 900, 256, 16),
+                                         (16, 1, 1500, 64, 300)])
+def test_subnormal_probabilities_are_kept(hq, hk, n, d, w):
+    """Logits 0 for the first key and -75 to -99.75 for the others: probabilities of 2^-108 to 2^-144,
+    two thirds of them below the smallest normal float. Bound: 2^-15 relative (the exponent's product
+    by log2 e, up to 144, is rounded to 2^-17, its factor to 2^-25; v_exp_f32 and the reciprocal are
+    far below that), one unit of 2^-149 for each row's two roundings and one for the mean."""
+    print(f"snap_scores subnormals hq={hq} hk={hk} n={n} d={d} w={w}", flush=True)
+    steps = 75 + 0.25 * (torch.arange(n) % 100).float()
+    steps[0] = 0
+    q = torch.zeros((1, hq, n, d), dtype=torch.float16)
+    k = torch.zeros((1, hk, n, d), dtype=torch.float16)
+    q[..., 0] = 8.0                                               # products by 8 are exact
+    k[..., 0] = -(steps * d ** 0.5 / 8).to(torch.float16)
+    got = snap_scores(q.cuda(), k.cuda(), w)
+    torch.cuda.synchronize()
+    logits = 8.0 * k[0, 0, :, 0].double() * d ** -0.5
+    visible = torch.arange(n)[None, :] <= torch.arange(n - w, n)[:, None]
+    p = torch.exp(logits)[None, :] * visible
+    ref = (p / p.sum(1, keepdim=True)).sum(0)
+    bound = 2.0 ** -15 * ref + (w + 1) * 2.0 ** -149
+    err = (got.cpu().double() - ref).abs()
+    assert (err <= bound).all(), float((err / bound).max())
+    assert (got[..., :n - w] > 0).all()
