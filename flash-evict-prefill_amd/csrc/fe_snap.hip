@@ -46,6 +46,13 @@ constexpr int kSnapLdsRows = 2048;   // rows per group whose statistics a scores
 // merging them all.
 constexpr int kSnapMergeMax = 16384;
 
+// Row tiles of partials up to which each key block has its own (16 MiB): every window of at most 128
+// rows to 131072 keys, or of 1024 rows to 32768, at 32/8 heads. Rows x key blocks grow with the window
+// times the prompt (1.1 GB for 32768 rows and keys), so beyond it a partial covers several key blocks
+// and row parts keep the CUs busy: 25 MB and 31.3 ms there (31.0 with 1.1 GB), 18 MB and 14.0 ms (13.2 with 538 MB)
+// for 4096 rows and 131072 keys.
+constexpr long long kSnapPartTiles = 65536;
+
 struct SnapArgs {
   const u16* q;
   const u16* k;
@@ -55,8 +62,9 @@ struct SnapArgs {
   long long qs[4], ks[4];
   int N, D, G, Hkv, BH;
   int W, R, RT, Rp;      // window rows per head, rows per group (G*W), 32-row tiles, 32 * RT
-  int S;                 // key blocks per (b, kv head)
-  int KG;                // key groups (of KT 32-key halves) per block
+  int NB, KG;            // key blocks per (b, kv head), key groups (of KT 32-key halves) per block
+  int S, per;            // partials per (b, kv head), each of `per` consecutive key blocks
+  int part_tiles;        // row tiles of a statistics block (all of a group's, or some chunks)
   float scale_log2;      // D^-0.5 * log2 e
 };
 
@@ -182,60 +190,65 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_stats_kernel(const S
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kg = wv % a.KG, rp = wv / a.KG, RP = NW / a.KG;
-  const int bh = (int)(blockIdx.x % (unsigned)a.BH), blk = (int)(blockIdx.x / (unsigned)a.BH);
+  const int bh = (int)(blockIdx.x % (unsigned)a.BH), idx = (int)(blockIdx.x / (unsigned)a.BH);
+  const int part = idx % a.S, rt_lo = idx / a.S * a.part_tiles, rt_hi = min(a.RT, rt_lo + a.part_tiles);
   const int b = bh / a.Hkv, hkv = bh - b * a.Hkv;
-  const int kb = (blk * a.KG + kg) * 32 * KT;
   const u16* kbase = a.k + b * a.ks[0] + hkv * a.ks[1];
 
-  u32x4 kf[KT][NDC];                              // K fragments (A operand) of the wave's keys
+  for (int blk = part * a.per; blk < min(a.NB, (part + 1) * a.per); ++blk) {
+    const int kb = (blk * a.KG + kg) * 32 * KT;
+    u32x4 kf[KT][NDC];                            // K fragments (A operand) of the wave's keys
 #pragma unroll
-  for (int s = 0; s < KT; ++s)
-    snap_load_keys<DP, VEC>(a, kbase, kb + 32 * s, rows + wv * 32 * (DP / 8), kf[s]);
-  __syncthreads();
-  const bool masked = kb + 32 * KT > a.N - a.W;   // some key of the wave is past some row
-  for (int rt0 = 0; rt0 < a.RT; rt0 += kSnapChunk) {
-    snap_load_rows<DP, VEC, 64 * NW>(a, b, hkv, rt0, rows);
+    for (int s = 0; s < KT; ++s)
+      snap_load_keys<DP, VEC>(a, kbase, kb + 32 * s, rows + wv * 32 * (DP / 8), kf[s]);
     __syncthreads();
-    for (int rt = rt0 + rp; rt < min(rt0 + kSnapChunk, a.RT); rt += RP) {
-      f32x16 x[KT];
+    const bool masked = kb + 32 * KT > a.N - a.W;   // some key of the wave is past some row
+    for (int rt0 = rt_lo; rt0 < rt_hi; rt0 += kSnapChunk) {
+      snap_load_rows<DP, VEC, 64 * NW>(a, b, hkv, rt0, rows);
+      __syncthreads();
+      for (int rt = rt0 + rp; rt < min(rt0 + kSnapChunk, rt_hi); rt += RP) {
+        f32x16 x[KT];
 #pragma unroll
-      for (int c = 0; c < NDC; ++c) {
-        const u32x4 qf = snap_frag<DP>(rows, (rt - rt0) * 32 + l32, 2 * c + hh);
+        for (int c = 0; c < NDC; ++c) {
+          const u32x4 qf = snap_frag<DP>(rows, (rt - rt0) * 32 + l32, 2 * c + hh);
 #pragma unroll
-        for (int s = 0; s < KT; ++s)
-          x[s] = c == 0 ? E::mfma(kf[s][0], qf, (f32x16){}) : E::mfma(kf[s][c], qf, x[s]);
-      }
-      // lanes hold query row rt*32 + l32; register i of half s holds key kb + 32s + 8(i/4) + 4h + i%4
-      float m = NEG_INF, l = 0.f;
-#pragma unroll
-      for (int s = 0; s < KT; ++s) {
-        round_logits<E>(x[s]);
-        if (masked) {
-          const int rel = snap_qpos(a, rt * 32 + l32) - kb - 32 * s - 4 * hh;
-#pragma unroll
-          for (int i = 0; i < 16; ++i) x[s][i] = 8 * (i >> 2) + (i & 3) <= rel ? x[s][i] : NEG_INF;
+          for (int s = 0; s < KT; ++s)
+            x[s] = c == 0 ? E::mfma(kf[s][0], qf, (f32x16){}) : E::mfma(kf[s][c], qf, x[s]);
         }
+        // lanes hold query row rt*32 + l32; register i of half s holds key kb + 32s + 8(i/4) + 4h + i%4
+        float m = NEG_INF, l = 0.f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) m = fmaxf(m, x[s][i]);
+        for (int s = 0; s < KT; ++s) {
+          round_logits<E>(x[s]);
+          if (masked) {
+            const int rel = snap_qpos(a, rt * 32 + l32) - kb - 32 * s - 4 * hh;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[s][i] = 8 * (i >> 2) + (i & 3) <= rel ? x[s][i] : NEG_INF;
+          }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) m = fmaxf(m, x[s][i]);
+        }
+        m = half_swap_max(m);
+        const float ref = snap_ref(m);
+#pragma unroll
+        for (int s = 0; s < KT; ++s) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) l += snap_exp(a, x[s][i] - ref);
+        }
+        l = half_swap_sum(l);
+        if (hh == 0) sm[kg][(rt - rt0) * 32 + l32] = make_float2(m, l);
       }
-      m = half_swap_max(m);
-      const float ref = snap_ref(m);
-#pragma unroll
-      for (int s = 0; s < KT; ++s) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) l += snap_exp(a, x[s][i] - ref);
+      __syncthreads();
+      const int nrows = min(kSnapChunk, rt_hi - rt0) * 32;
+      for (int r = tid; r < nrows; r += 64 * NW) {
+        float m = sm[0][r].x, l = sm[0][r].y;
+        for (int g = 1; g < a.KG; ++g) snap_merge(a, m, l, sm[g][r].x, sm[g][r].y);
+        float2* out = a.part + ((long long)bh * a.S + part) * a.Rp + rt0 * 32 + r;
+        if (blk > part * a.per) snap_merge(a, m, l, out->x, out->y);   // this thread's own of the block before
+        *out = make_float2(m, l);
       }
-      l = half_swap_sum(l);
-      if (hh == 0) sm[kg][(rt - rt0) * 32 + l32] = make_float2(m, l);
+      __syncthreads();
     }
-    __syncthreads();
-    const int nrows = min(kSnapChunk, a.RT - rt0) * 32;
-    for (int r = tid; r < nrows; r += 64 * NW) {
-      float m = sm[0][r].x, l = sm[0][r].y;
-      for (int g = 1; g < a.KG; ++g) snap_merge(a, m, l, sm[g][r].x, sm[g][r].y);
-      a.part[((long long)bh * a.S + blk) * a.Rp + rt0 * 32 + r] = make_float2(m, l);
-    }
-    __syncthreads();
   }
 }
 
@@ -449,6 +462,13 @@ int snap_split(long long BH, long long N, int waves, int& KG, int& KT) {
   return (int)blocks();
 }
 
+// Partials per (b, kv head): one per key block, fewer where they would exceed kSnapPartTiles row tiles.
+int snap_parts(long long BH, long long NB, long long RT) {
+  const long long tiles = BH * RT;
+  if (tiles < 1 || tiles > kSnapPartTiles) return 1;   // below 1: sizes past 64 bits, refused by the call
+  return (int)(NB < kSnapPartTiles / tiles ? NB : kSnapPartTiles / tiles);
+}
+
 bool snap_vec(const void* p, const int64_t* st, int64_t D) {
   return st[3] == 1 && D % 8 == 0 && ((uintptr_t)p % 16) == 0 && st[0] % 8 == 0 && st[1] % 8 == 0 &&
          st[2] % 8 == 0;
@@ -463,7 +483,7 @@ extern "C" size_t fe_snap_scores_workspace_bytes(int64_t B, int64_t Hq, int64_t 
   const long long W = window < N ? window : N;
   const long long BH = B * Hkv, R = (Hq / Hkv) * W, RT = (R + 31) / 32;
   int KG, KT;
-  const int S = snap_split(BH, N, snap_waves(256), KG, KT);   // the most blocks of any head dim
+  const int S = snap_parts(BH, snap_split(BH, N, snap_waves(256), KG, KT), RT);   // the most of any head dim
   return (size_t)(BH * RT * 32) * sizeof(float2) * (size_t)(S + 1);
 }
 
@@ -499,7 +519,15 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
     return FE_ERR_UNSUPPORTED;
   }
   int KG, KT;
-  const int waves = snap_waves(D <= 128 ? 128 : 256), S = snap_split(BH, N, waves, KG, KT);
+  const int waves = snap_waves(D <= 128 ? 128 : 256), NB = snap_split(BH, N, waves, KG, KT);
+  const int most = snap_parts(BH, NB, RT), per = (NB + most - 1) / most, S = (NB + per - 1) / per;
+  // statistics blocks: one per partial, or, where a partial covers several key blocks, row parts (of whole
+  // chunks) to make 1024 blocks. Fewer read K less often: with 512, 1% less.
+  const long long chunks = (RT + kSnapChunk - 1) / kSnapChunk;
+  long long RS = 1;
+  if (per > 1) RS = (1024 + BH * S - 1) / (BH * S);
+  const long long part_chunks = (chunks + (RS < chunks ? RS : chunks) - 1) / (RS < chunks ? RS : chunks);
+  RS = (chunks + part_chunks - 1) / part_chunks;
   const size_t need = fe_snap_scores_workspace_bytes(B, Hq, Hkv, N, window);
   if (!workspace || workspace_bytes < need) {
     set_error("fe_snap_scores: needs a workspace of fe_snap_scores_workspace_bytes() bytes");
@@ -524,8 +552,11 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
   a.R = (int)R;
   a.RT = (int)RT;
   a.Rp = (int)(RT * 32);
-  a.S = S;
+  a.NB = NB;
   a.KG = KG;
+  a.S = S;
+  a.per = per;
+  a.part_tiles = (int)(part_chunks * kSnapChunk);
   a.scale_log2 = (float)(1.4426950408889634 * pow((double)D, -0.5));
   const int vec = snap_vec(q, q_strides, D) && snap_vec(k, k_strides, D) ? 1 : 0;
   const int bf = dtype == FE_DTYPE_BF16 ? 1 : 0;
@@ -534,13 +565,13 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
   const void* scores_fn = kSnapKernels[ki + 1].fn;
   hipStream_t stream = (hipStream_t)hip_stream;
   void* kargs[] = {&a};
-  const dim3 grid((unsigned)(BH * S)), block(64 * waves);
-  hipError_t err = hipLaunchKernel(stats_fn, grid, block, kargs, 0, stream);
+  const dim3 block(64 * waves);
+  hipError_t err = hipLaunchKernel(stats_fn, dim3((unsigned)(BH * S * RS)), block, kargs, 0, stream);
   if (err == hipSuccess && a.stats) {
     const long long rows = BH * RT * 32;
     err = hipLaunchKernel((const void*)snap_combine_kernel, dim3((unsigned)(rows / 32)), dim3(1024), kargs, 0, stream);
   }
-  if (err == hipSuccess) err = hipLaunchKernel(scores_fn, grid, block, kargs, 0, stream);
+  if (err == hipSuccess) err = hipLaunchKernel(scores_fn, dim3((unsigned)(BH * NB)), block, kargs, 0, stream);
   if (err != hipSuccess) {
     set_error(std::string("fe_snap_scores: launch: ") + hipGetErrorString(err));
     return FE_ERR_HIP;

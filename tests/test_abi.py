@@ -141,3 +141,22 @@ def test_workspace_sizer_adds_repack_room_only_for_layouts_the_fast_kernels_cann
         assert size(100, 4096, (Hkv * N * 100, N * 100, 100, 1), vst=(Hkv * N * 100, N * 100, 100, 1),
                     score=score) == base + repack(100)
         assert size(128, 4096, (Hkv * N * 128, N * 128, 128, 1), vptr=4100, score=score) == base + repack(128)
+
+
+def test_snap_workspace_is_bounded_at_wide_windows():
+    """At most 16 MiB of partials, or one per row where that is more, and the merged rows; the row counts
+    of the shapes a model has. A window of the whole prompt takes 16 bytes a row."""
+    L = _lib.lib()
+
+    def rows(b, hq, hk, n, w):
+        return b * hk * (((hq // hk) * min(w, n) + 31) // 32) * 32
+
+    for b, hq, hk in ((1, 4, 4), (1, 7, 1), (1, 28, 4), (1, 32, 8), (2, 64, 8), (16, 32, 8)):
+        for n in (1, 31, 512, 1531, 8192, 32768, 131072, 1 << 20):
+            for w in (1, 32, 128, 1024, 4096, n):
+                size, r = L.fe_snap_scores_workspace_bytes(b, hq, hk, n, w), rows(b, hq, hk, n, w)
+                assert 16 * r <= size <= max(16 << 20, 8 * r) + 8 * r, (b, hq, hk, n, w, size)
+    assert L.fe_snap_scores_workspace_bytes(1, 32, 8, 131072, 131072) == 16 * 32 * 131072
+    assert L.fe_snap_scores_workspace_bytes(1, 32, 8, 131072, 4096) <= 18 << 20
+    # sizes whose products pass 64 bits: a size, and no trap (the call itself refuses them)
+    assert L.fe_snap_scores_workspace_bytes(1 << 40, 1 << 40, 1 << 40, 1 << 40, 1 << 40) >= 0

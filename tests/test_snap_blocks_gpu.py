@@ -1,6 +1,7 @@
 """fe_snap_scores over its block shapes: key groups per block (8 down to 1, by the key count),
 64 or 32 keys per group, row parts, more than one chunk of row tiles per block, and windows of
-more rows per group than a block keeps statistics of (the combine kernel). Against the oracle,
+more rows per group than a block keeps statistics of (the combine kernel), up to those whose partials
+cover several key blocks. Against the oracle,
 with the tolerance of test_snap_gpu (a logit near a rounding boundary may land one ulp of the
 input type apart)."""
 import pytest
@@ -23,6 +24,9 @@ pytestmark = pytest.mark.gpu
     (1, 8, 8, 16500, 256, 20, torch.bfloat16, "contiguous"),     # tile dim 256: four waves
     (1, 16, 1, 700, 64, 300, torch.bfloat16, "contiguous"),      # 4800 rows per group: combine kernel, three LDS loads
     (1, 16, 2, 400, 72, 256, torch.float16, "channel_stride2"),  # exactly 2048 rows, element loads
+    (1, 32, 1, 1536, 64, 1536, torch.bfloat16, "contiguous"),    # 1536 row tiles: 2 key blocks per partial, row parts
+    (1, 20, 1, 1999, 200, 1999, torch.float16, "transposed"),    # 2 of 63 key blocks per partial, rows ragged, four waves
+    (2, 64, 1, 1100, 32, 1100, torch.bfloat16, "transposed"),    # 3 key blocks per partial, 2 in the last
 ])
 def test_snap_block_shapes_match_oracle(b, hq, hk, n, d, w, dtype, layout):
     print(f"snap_scores blocks b={b} hq={hq} hk={hk} n={n} d={d} w={w} {dtype} {layout}", flush=True)
