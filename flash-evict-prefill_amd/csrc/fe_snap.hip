@@ -49,8 +49,8 @@ constexpr int kSnapMergeMax = 16384;
 // Row tiles of partials up to which each key block has its own (16 MiB): every window of at most 128
 // rows to 131072 keys, or of 1024 rows to 32768, at 32/8 heads. Rows x key blocks grow with the window
 // times the prompt (1.1 GB for 32768 rows and keys), so beyond it a partial covers several key blocks
-// and row parts keep the CUs busy: 25 MB and 31.3 ms there (31.0 with 1.1 GB), 18 MB and 14.0 ms (13.2 with 538 MB)
-// for 4096 rows and 131072 keys.
+// and row parts keep the CUs busy: 25 MB and 23.2 ms there (28.5 with 1.1 GB and no key block left out), 18 MB and
+// 14.0 ms (13.2 with 538 MB) for 4096 rows and 131072 keys.
 constexpr long long kSnapPartTiles = 65536;
 
 struct SnapArgs {
@@ -154,6 +154,11 @@ __device__ __forceinline__ int snap_qpos(const SnapArgs& a, int r) {
   return r < a.R ? a.N - a.W + r % a.W : -1;
 }
 
+// Largest position among the group's rows r0 .. r1 (r1 below R).
+__device__ __forceinline__ int snap_last(const SnapArgs& a, int r0, int r1) {
+  return r0 / a.W == r1 / a.W ? a.N - a.W + r1 % a.W : a.N - 1;
+}
+
 // exp(scale * x) for x <= 0, a difference of two rounded logits (exact in FP32 unless one is
 // 2^13 times the other): one product by scale * log2 e and v_exp_f32. Against 64 bits the scores
 // are as close as with expf(scale * logit - scale * max): 7.3e-7 to 3.6e-6 relative over ten shapes
@@ -195,7 +200,10 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_stats_kernel(const S
   const int b = bh / a.Hkv, hkv = bh - b * a.Hkv;
   const u16* kbase = a.k + b * a.ks[0] + hkv * a.ks[1];
 
-  for (int blk = part * a.per; blk < min(a.NB, (part + 1) * a.per); ++blk) {
+  // key blocks up to the last of the part's rows (one at least, which writes the partial)
+  int blk_hi = min(a.NB, (part + 1) * a.per);
+  if (a.per > 1) blk_hi = max(part * a.per + 1, min(blk_hi, snap_last(a, rt_lo * 32, min(rt_hi * 32, a.R) - 1) / (a.KG * 32 * KT) + 1));
+  for (int blk = part * a.per; blk < blk_hi; ++blk) {
     const int kb = (blk * a.KG + kg) * 32 * KT;
     u32x4 kf[KT][NDC];                            // K fragments (A operand) of the wave's keys
 #pragma unroll
@@ -326,6 +334,7 @@ __global__ __launch_bounds__(64 * snap_waves(DP)) void snap_scores_kernel(const 
       // statistics of rows r0 .. r0 + rows - 1 into LDS
       const int rows = min(kSnapLdsRows, a.Rp - r0);
       if (a.stats) {
+        if (snap_last(a, r0, min(r0 + rows, a.R) - 1) < blk * a.KG * 32 * KT) continue;   // keys past all of them
         if (r0 > 0) __syncthreads();
         for (int r = tid; r < rows; r += NT) {
           const float2 v = a.stats[(long long)bh * a.Rp + r0 + r];
@@ -522,7 +531,8 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
   const int waves = snap_waves(D <= 128 ? 128 : 256), NB = snap_split(BH, N, waves, KG, KT);
   const int most = snap_parts(BH, NB, RT), per = (NB + most - 1) / most, S = (NB + per - 1) / per;
   // statistics blocks: one per partial, or, where a partial covers several key blocks, row parts (of whole
-  // chunks) to make 1024 blocks. Fewer read K less often: with 512, 1% less.
+  // chunks) to make 1024 blocks. Fewer read K less often and end later: with 512 a window of 1024 rows
+  // takes 1% less, one of 32768 rows 16% more.
   const long long chunks = (RT + kSnapChunk - 1) / kSnapChunk;
   long long RS = 1;
   if (per > 1) RS = (1024 + BH * S - 1) / (BH * S);

@@ -26,6 +26,7 @@ pytestmark = pytest.mark.gpu
     (1, 16, 2, 400, 72, 256, torch.float16, "channel_stride2"),  # exactly 2048 rows, element loads
     (1, 32, 1, 1536, 64, 1536, torch.bfloat16, "contiguous"),    # 1536 row tiles: 2 key blocks per partial, row parts
     (1, 20, 1, 1999, 200, 1999, torch.float16, "transposed"),    # 2 of 63 key blocks per partial, rows ragged, four waves
+    (1, 2, 1, 6001, 64, 6001, torch.bfloat16, "contiguous"),     # rows whose last position is before a block's keys
     (2, 64, 1, 1100, 32, 1100, torch.bfloat16, "transposed"),    # 3 key blocks per partial, 2 in the last
 ])
 def test_snap_block_shapes_match_oracle(b, hq, hk, n, d, w, dtype, layout):
