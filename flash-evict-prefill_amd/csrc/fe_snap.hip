@@ -100,6 +100,15 @@ __device__ __forceinline__ u32x4 snap_frag(const u32x4* rows, int r, int ch) {
   return rows[r * (DP / 8) + (ch ^ snap_swz<DP>(r))];
 }
 
+// Orders a wave's LDS accesses before and after it for lanes that read each other's data. The hardware
+// completes them in order, so this emits no wait of its own; it keeps the compiler, which sees one
+// thread's addresses only, from moving a lane's loads above its stores or its next stores above them.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // The wave's K fragments of keys kb .. kb+31 through its own 32 rows of LDS (zeros past N).
 template <int DP, int VEC>
 __device__ __forceinline__ void snap_load_keys(const SnapArgs& a, const u16* kbase, int kb, u32x4* rows, u32x4 (&f)[DP / 16]) {
@@ -118,10 +127,10 @@ __device__ __forceinline__ void snap_load_keys(const SnapArgs& a, const u16* kba
     const int i = lane + 64 * j;
     rows[(i / CPR) * CPR + ((i % CPR) ^ snap_swz<DP>(i / CPR))] = v[j];
   }
-  // one wave's LDS operations complete in order: the reads below see the writes above, and the
-  // next call's writes come after these reads
+  wave_lds_order();
 #pragma unroll
   for (int c = 0; c < DP / 16; ++c) f[c] = snap_frag<DP>(rows, lane & 31, 2 * c + (lane >> 5));
+  wave_lds_order();   // the next call writes these rows
 }
 
 // Row tiles rt0 .. rt0 + kSnapChunk - 1 of the group's query rows into LDS by the whole block
