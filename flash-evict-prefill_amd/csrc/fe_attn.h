@@ -34,7 +34,7 @@ struct AttnArgs {
   int nitems;                       // dynamic schedule: work items of the launch
   int nstatic;                      // dynamic schedule: workgroups launched (each starts with item blockIdx.x)
   int tail;                         // dynamic schedule: first item of the queues' light parts (nitems: none)
-  int nattn;                        // attention items; items past them are replay items
+  int nattn;                        // attention items; items past them are replay items (kReplayItemMaxDim)
   int rwg0;                         // replay items in ascending row groups from rwg0 (-1: heaviest first)
   unsigned* done;                   // replay items: one bit per attention item, set once its biases are out
   int wait_base, wait_per_tile;     // replay items: polls of a dependency's bit (plus per key tile) before running it
@@ -54,6 +54,10 @@ constexpr int kQueueDone = 2 * kQueueReplay;
 constexpr int kMaxDoneItems = 16384;
 constexpr int kQueueWords = kQueueDone + kMaxDoneItems / 32;
 constexpr size_t kQueueBytes = kQueueWords * sizeof(int);
+// Largest tile dim whose attention kernels hold replay items' code: above it that code cost the tile loop
+// registers. A launch makes items for no other kernel, which would take them for attention items of a
+// negative row group.
+constexpr int kReplayItemMaxDim = 128;
 // s_getreg_b32 operand of hwreg(HW_REG_XCC_ID): register 20, bits 0-31 (the XCC index is bits 0-3)
 constexpr int kHwRegXccId = (31 << 11) | 20;
 

@@ -712,6 +712,7 @@ int64_t one_shot_grid(int64_t items) { return items + ((items / 8 + 7) & ~(int64
 #ifndef FE_SMALL_LAUNCH_MAX_D
 #define FE_SMALL_LAUNCH_MAX_D 128
 #endif
+static_assert(FE_SMALL_LAUNCH_MAX_D <= kReplayItemMaxDim, "replay items only where the attention kernel has their code");
 // Tail replay items on fused_fast_kernel too (build option: the reference harness's shape at
 // 32K 3% faster with them; D = 64 at the headline head counts within run-to-run drift).
 #ifndef FE_TAIL_FAST

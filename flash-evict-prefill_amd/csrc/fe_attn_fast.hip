@@ -327,7 +327,7 @@ __global__ __launch_bounds__(NW * 64, (FastOccupancy<NW, DP>::WAVES_PER_EU)) voi
   constexpr int SLOTS = (DP <= 128 && !FastOccupancy<NW, DP>::SMALL_GRID) ? 2 : 1;
   // replay items: the launch makes none for 12 waves, nor above tile dim 128, where their code beside
   // the attention items' cost the tile loop registers
-  constexpr bool ITEMS = NW <= 8 && DP <= 128;
+  constexpr bool ITEMS = NW <= 8 && DP <= kReplayItemMaxDim;
   constexpr bool PIPE = FastOccupancy<NW, DP>::SMALL_GRID && DP > 64;   // tile loop: pipe_loop
   static_assert(NDC % KH == 0, "K fragment groups");
   static_assert(NW % 2 == 0 && NW >= 4, "row tiles per workgroup");

@@ -3,6 +3,8 @@ before touching a GPU (CPU-only checks: no device compute is launched here)."""
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 
@@ -160,3 +162,17 @@ def test_snap_workspace_is_bounded_at_wide_windows():
     assert L.fe_snap_scores_workspace_bytes(1, 32, 8, 131072, 4096) <= 18 << 20
     # sizes whose products pass 64 bits: a size, and no trap (the call itself refuses them)
     assert L.fe_snap_scores_workspace_bytes(1 << 40, 1 << 40, 1 << 40, 1 << 40, 1 << 40) >= 0
+
+
+@pytest.mark.parametrize("define,ok", [((), True), (("-DFE_SMALL_LAUNCH_MAX_D=256",), False)])
+def test_replay_items_only_for_kernels_that_hold_their_code(define, ok):
+    """The launch's limit for replay items may not be built above the kernels' (host pass only, about a
+    second): items past it would index row groups below zero."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    src = os.path.join(ROOT, "flash-evict-prefill_amd", "csrc", "fe_attn.hip")
+    r = subprocess.run([hipcc, "--offload-arch=gfx950", "-std=c++17", "--cuda-host-only", "-fsyntax-only", *define, src],
+                       capture_output=True, text=True)
+    assert (r.returncode == 0) == ok, r.stderr
+    assert ok or "static assertion failed" in r.stderr
