@@ -532,7 +532,8 @@ extern "C" int fe_snap_scores(const void* q, const void* k, float* scores, int64
     }
   const long long W = window < N ? window : N;
   const long long G = Hq / Hkv, BH = B * Hkv, R = G * W, RT = (R + 31) / 32;
-  if (N > (1LL << 30) || R > (1LL << 30) || BH * RT * 32 > (1LL << 40) || BH * ((N + 31) / 32) > 0x7fffffffLL) {
+  // each grid within 31 bits: at most one block per 64 keys or per row tile (32 keys only below 256 blocks)
+  if (N > (1LL << 30) || R > (1LL << 30) || BH * RT > 0x7fffffffLL || BH * ((N + 63) / 64) > 0x7fffffffLL) {
     set_error("fe_snap_scores: problem too large");
     return FE_ERR_UNSUPPORTED;
   }

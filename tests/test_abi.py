@@ -14,6 +14,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "flash_evict.h")
 
 FE_ERR_INVALID = -1
+FE_ERR_UNSUPPORTED = -4
 FE_ERR_WORKSPACE = -3
 
 
@@ -176,3 +177,19 @@ def test_replay_items_only_for_kernels_that_hold_their_code(define, ok):
                        capture_output=True, text=True)
     assert (r.returncode == 0) == ok, r.stderr
     assert ok or "static assertion failed" in r.stderr
+
+
+def test_snap_scores_refuses_grids_past_31_bits_and_nothing_smaller():
+    """Row tiles, and 64-key tiles, times (batch, KV head) pairs, up to 2^31 - 1; checked before the
+    workspace is, and before any launch."""
+    L = _lib.lib()
+    st = (ctypes.c_int64 * 4)(1, 1, 1, 1)
+    p = ctypes.c_void_p(16)
+
+    def call(hkv, g, n, w):
+        return L.fe_snap_scores(p, p, p, 1, hkv * g, hkv, n, 64, st, st, 1, w, None, 0, None)
+
+    assert call(1 << 26, 64, 32, 32) == FE_ERR_UNSUPPORTED          # 64 row tiles each: 2^32
+    assert call(1 << 25, 63, 32, 32) == FE_ERR_WORKSPACE            # 63 x 2^25
+    assert call((1 << 30) + 1, 1, 64, 1) == FE_ERR_WORKSPACE        # one 64-key tile each
+    assert call((1 << 30) + 1, 1, 65, 1) == FE_ERR_UNSUPPORTED      # two
