@@ -46,8 +46,8 @@ struct AttnArgs {
 // on its own 128-byte line, the attention kernel's from word 0 and the replay kernel's from
 // word kQueueReplay; a queue's counters are the 64-bit words at ints 0 and 2 of its line (its
 // heavy and light parts, take_item in fe_attn_fast.hip). Then, from word kQueueDone, one bit per
-// attention item for the replay items of attn_rt2_kernel (kMaxDoneItems bits). Zeroed before
-// every launch.
+// attention item for the replay items of either attention kernel (kMaxDoneItems bits; consecutive items
+// on different lines, done_word in fe_attn_fast.hip). Zeroed before every launch.
 constexpr int kQueueStride = 32;
 constexpr int kQueueReplay = 8 * kQueueStride;
 constexpr int kQueueDone = 2 * kQueueReplay;
@@ -101,7 +101,7 @@ struct ReplayPlan {
   int rows;
   const char* name;
 };
-// The small-grid attention kernel at tile dims 32 and 64 (4-wave workgroups), where it applies.
+// The small-grid attention kernel (4-wave workgroups) at tile dims 32 to 128, where it applies.
 bool fast_plan_small(const AttnArgs& a, int dtype, FusedPlan& plan);
 bool replay_plan(const AttnArgs& a, int dtype, ReplayPlan& plan);
 hipError_t prepare_plan(const FusedPlan& plan);

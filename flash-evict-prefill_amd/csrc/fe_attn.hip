@@ -705,7 +705,7 @@ int64_t one_shot_grid(int64_t items) { return items + ((items / 8 + 7) & ~(int64
 #ifndef FE_REPLAY_ITEMS_PER_WG
 #define FE_REPLAY_ITEMS_PER_WG 2
 #endif
-// Key tiles a replay item holds at least (where the rows' keys allow).
+// All the replay of small causal launches as items, up to this tile dim.
 #ifndef FE_SMALL_LAUNCH_ITEMS
 #define FE_SMALL_LAUNCH_ITEMS 1
 #endif
@@ -723,6 +723,8 @@ static_assert(FE_SMALL_LAUNCH_MAX_D <= kReplayItemMaxDim, "replay items only whe
 #ifndef FE_REPLAY_ROUNDS_SPLIT
 #define FE_REPLAY_ROUNDS_SPLIT 1
 #endif
+// Key tiles a replay item holds at least (where the rows' keys allow): FE_SMALL_ITEM_MIN_TILES in small
+// causal launches with workgroups to spare, FE_REPLAY_ITEM_MIN_TILES elsewhere.
 #ifndef FE_SMALL_ITEM_MIN_TILES
 #define FE_SMALL_ITEM_MIN_TILES 2
 #endif
@@ -956,7 +958,7 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
   // kernel's row tiles holding window rows, key range): key ranges chosen for about two items per
   // resident workgroup (four measured 1.3% slower at llama8k), of at least
   // FE_REPLAY_ITEM_MIN_TILES key tiles where the keys allow (a window of 128 rows at N = 32K
-  // otherwise made items of two tiles, 0.4% slower overall).
+  // otherwise made items of two tiles, 0.4% slower overall); small causal launches go below that (below).
   bool replay_items = false;
   // Causal launches at tile dims up to 128 whose attention items do not fill the resident
   // workgroups: a grid of every resident workgroup, and all the replay as items in ascending row
@@ -975,9 +977,12 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
     rs = rs < 1 ? 1 : (rs > rs_max ? rs_max : rs);
     // With workgroups to spare, shorter key ranges, down to FE_SMALL_ITEM_MIN_TILES key tiles and up to
     // half the resident workgroups in items: the launch ends with the replay of the heaviest rows, all
-    // of it serial after their attention items. In more items than that the rows' Q, biases and waits
-    // cost more than the shorter ranges save (1050 rows of B1 Hq4/Hkv1 D64 N3323 in 884 items instead
-    // of 238: 1.4% slower).
+    // of it serial after their attention items; in more items than that the rows' Q, biases and waits
+    // cost more than the shorter ranges save. prefill(), us, with none / a quarter / half / three quarters /
+    // all of the resident workgroups: B1 Hq4/Hkv4 D64 N512 27.1 / 23.4 / 23.2 / 23.1 / 23.2, Hq8/Hkv2 D128 N1000
+    // 41.6 / 41.6 / 38.1 / 37.0 / 37.2, Hq4/Hkv2 D64 N2048 47.8 / 47.7 / 44.8 / 44.3 / 44.2, Hq32/Hkv8 D128 N512
+    // 33.3 / 33.4 / 30.8 / 30.6 / 30.5, Hq16/Hkv4 D64 N900 32.1 / 32.1 / 32.1 / 33.7 / 34.3, 1050 rows of Hq4/Hkv1
+    // D64 N3323 64.0 / 64.0 / 63.3 / 65.8 / 65.6; eight more shapes within 3% from half on.
     const int64_t spare = resident - items < resident / 2 ? resident - items : resident / 2;
     const int64_t free_rs = nwg > 0 ? spare / nwg : 0;
     const int64_t short_rs = (max_tiles + FE_SMALL_ITEM_MIN_TILES - 1) / FE_SMALL_ITEM_MIN_TILES;

@@ -24,8 +24,8 @@
 // and the latency of each step make the rest. Layout: a wave keeps the K fragments of its keys in
 // registers and runs over the row tiles, whose Q the block holds in LDS, eight tiles at a time. (One
 // row tile per wave against a strip of K, 64-thread blocks, read K once per row tile and left a combine
-// kernel of few threads with a serial loop over the strips: 47.6 + 37.2 + 35.0 us at 28/4 heads,
-// N = 32768, D = 128, window 32, against 19.0 + 23.6 us here.)
+// kernel of few threads with a serial loop over the strips: 47.9 + 37.1 + 35.3 us at 28/4 heads,
+// N = 32768, D = 128, window 32, against 18.6 + 23.8 us here.)
 #include <math.h>
 #include <string>
 
@@ -41,16 +41,18 @@ constexpr int snap_waves(int DP) { return DP > 128 ? 4 : 8; }
 constexpr int kSnapChunk = 8;        // row tiles between two merges of the key groups' partials
 constexpr int kSnapLdsRows = 2048;   // rows per group whose statistics a scores block keeps in LDS
 // Partials of a group up to which each scores block merges them itself (128 KiB through L2 a
-// block: about the 4.6 us of another launch). More go through snap_combine_kernel: B1 Hq7/Hkv1 D64
-// N = 40831, window 128 (319 x 896 partials), scores and selection 84 us, 211 with every block
-// merging them all.
+// block: about the 4.6 us of another launch). More go through snap_combine_kernel. Calls with a limit of
+// 4096 / 8192 / 16384 / 32768 / 131072 partials, us: Hq8/Hkv2 D64 N65536 window 16 19.1 / 17.2 / 17.3 / 17.3 /
+// 17.1, Hq28/Hkv4 D128 N32768 window 64 63.7 / 63.5 / 63.4 / 67.8 / 67.9, Hq32/Hkv8 N65536 window 64 157 / 156 / 157 /
+// 182 / 182, Hq14/Hkv2 D64 N30000 window 64 39 / 39 / 39 / 39 / 82; nine more shapes the same to 16384, and 0-18%
+// slower at 32768.
 constexpr int kSnapMergeMax = 16384;
 
 // Row tiles of partials up to which each key block has its own (16 MiB): every window of at most 128
 // rows to 131072 keys, or of 1024 rows to 32768, at 32/8 heads. Rows x key blocks grow with the window
 // times the prompt (1.1 GB for 32768 rows and keys), so beyond it a partial covers several key blocks
-// and row parts keep the CUs busy: 25 MB and 23.2 ms there (28.5 with 1.1 GB and no key block left out), 18 MB and
-// 14.0 ms (13.2 with 538 MB) for 4096 rows and 131072 keys.
+// and row parts keep the CUs busy: 25 MB and 23.2 ms there (28.5 with 1.1 GB and no key block left out), 18 MB
+// and 14.0 ms (13.2 with 538 MB) for 4096 rows and 131072 keys.
 constexpr long long kSnapPartTiles = 65536;
 
 struct SnapArgs {

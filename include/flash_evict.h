@@ -201,7 +201,8 @@ int fe_gather_rows(const void* x, const int64_t* indices, void* out,
  *   scores[b,j,n] = (1/G) * sum_{h in group j} sum_t p[h,t,n]
  * q: [B,Hq,N,D], k: [B,Hkv,N,D] with element strides {b,h,n,d}; scores: contiguous
  * [B,Hkv,N] float32, every element written. workspace: device memory of at least
- * fe_snap_scores_workspace_bytes(...) bytes. window >= 1.
+ * fe_snap_scores_workspace_bytes(...) bytes: at most 16 MiB, or 8 bytes per window row of every
+ * query head where that is more, and 8 more per row (rows of a group rounded up to 32). window >= 1.
  */
 size_t fe_snap_scores_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t N, int64_t window);
 int fe_snap_scores(const void* q, const void* k, float* scores, int64_t B, int64_t Hq, int64_t Hkv,
